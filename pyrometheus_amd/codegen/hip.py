@@ -40,6 +40,7 @@ numpy source, so results agree with the reference to rounding, not bitwise.
 
 from __future__ import annotations
 
+import decimal
 import math
 import os
 from typing import Dict, List, Optional, Sequence, Tuple
@@ -53,6 +54,9 @@ ABI_VERSION = 1
 #: mechanisms up to this many species also get the dense-Jacobian kernels
 #: (the NS x NS Jacobian lives in registers) and the flamelet kernels
 DENSE_JAC_MAX_SPECIES = 16
+LOG10_2 = math.log10(2.0)
+_DEC = decimal.Context(prec=40)
+_LN2 = _DEC.ln(decimal.Decimal(2))
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
                     "csrc")
 
@@ -104,7 +108,9 @@ class _Writer:
 #:  lazy  -- the omega-dot and JVP kernels open species (load C_k, compute
 #:           exp(g'_k)) at their first use and store each rate after its last
 #:           update, along a reaction order that keeps few species open
-#:           (``reaction_order``); ``order_tries`` greedy restarts;
+#:           (``reaction_order``); ``order_tries`` greedy restarts
+#:           (``wdot_tries`` for omega-dot: GRI-3.0's peak falls from 73 to
+#:           67 species values at the 21st, 2.40 -> 2.03 ms on 2^22 cells);
 #:  wdot_waves / deriv_waves -- waves per SIMD the compiler must budget
 #:           registers for in k_wdot / k_wdot_jvp (0: its own choice);
 #:  lazy_fence -- an empty asm with a memory clobber every that many
@@ -173,11 +179,25 @@ class _Writer:
 #:           GRI-3.0 cells, timed side by side);
 #:  nt_rq -- the same for the per-reaction outputs (k_f and the like: no
 #:           change measured, off).
+#:  base2 -- the lazy omega-dot pass takes the powers of its exponents with
+#:           pyro::exp2p / expp (15 and 17 VALU operations) instead of exp
+#:           (about 25), writes Troe's blending in base-2 logarithms (one log2
+#:           per reaction beside one per shared [M], k_inf's power merged
+#:           with F's) and forms [M] sums that several reactions share once
+#:           per cell: 19,910 -> 12,965 VALU operations per wave;
+#:  wdot_ctable -- that pass reads its constants from one table through
+#:           scalar loads instead of literals.  Off: each reaction waits for
+#:           its loads, which a full chip hides and a partly filled one does
+#:           not (16,384 GRI-3.0 cells 56 against 40 us, 131,072 cells 88
+#:           against 69 us, 2^22 cells 2.02 against 2.00 ms);
 #: (GRI-3.0, 2^24 cells: 16.6 ms with the species arrays held in registers,
-#: 12.1 ms lazy at two waves per SIMD, 11.35 ms with zform.)
+#: 12.1 ms lazy at two waves per SIMD, 11.35 ms with zform, 7.8 ms with
+#: base2.  What bounds it there is FP64 issue at the clock that the card
+#: holds under it: an independent FP64 operation takes 2.2 ns per SIMD with
+#: every SIMD busy, 13k of them 1.8 of the 2.0 ms of 2^22 cells.)
 DEFAULT_TUNING = {"pin": True, "pin_every": 3, "kc": "species", "ctable": True,
                   "lazy": True, "wdot_waves": 2, "deriv_waves": 0,
-                  "lazy_fence": 1, "order_tries": 8, "prefetch": 4,
+                  "lazy_fence": 1, "order_tries": 8, "wdot_tries": 21, "prefetch": 4,
                   "zform": True, "jac_groups": 4, "ystash": 39}
 
 
@@ -236,10 +256,16 @@ class _Lowering:
         self.tab = None  # list of tabulated constants while emitting a table
         # value -> index into tab, when constants are shared while emitting
         self.tab_index = None
-        # exp of the Arrhenius and Gibbs exponents (bounded arguments)
+        # the power taken of the Arrhenius and of the Gibbs exponents
         self.fexp = "exp"
+        self.gexp = "exp"
         # reciprocal in K_c^-1 (products of Gibbs factors)
         self.frecip = "pyro::recip"
+        # Arrhenius and Gibbs exponents in base 2 (constants scaled by
+        # log2(e)) and their powers from pyro::exp2p
+        self.base2 = False
+        # efficiency key -> ([M], log2 [M]) variables, formed once per cell
+        self.m_shared = {}
         # K_c^-1 from E[] of the products and F[] = 1 / E[] of the
         # reactants (set while emitting the lazy derivative passes)
         self.kinv_f = False
@@ -261,6 +287,34 @@ class _Lowering:
             return f"K[{j}]"
         self.tab.append(x)
         return f"K[{len(self.tab) - 1}]"
+
+    def exponent(self, b: float, ta: float, ln_a) -> str:
+        """b ln T - Ta/T + ln A in the current base, each constant rounded
+        once.  In base 2 the constants b log2(e) and Ta log2(e) are no
+        longer the mechanism's own decimals; what their rounding leaves at
+        1200 K is put into the third, which keeps the exponent's error at
+        that of the base-e form (GRI-3.0 over 300..2500 K: 2.4e-15 rms
+        against 2.5e-15; 2.6e-15 without)."""
+        D = decimal.Decimal
+        if not self.base2:
+            inner = (self.c(float(ln_a)) if ta == 0 else
+                     f"fma({self.c(-ta)}, invT, {self.c(float(ln_a))})")
+            return inner if b == 0 else f"fma({self.c(b)}, lnT, {inner})"
+        t0 = D(1200)
+        bx, tx, ax = (_DEC.divide(x, _LN2) for x in (D(b), D(ta), ln_a))
+        b2, t2 = float(bx), float(tx)
+        a2 = self.c(float(ax + (bx - D(b2)) * _DEC.ln(t0)
+                          - _DEC.divide(tx - D(t2), t0)))
+        if t2 == 0:
+            return a2 if b2 == 0 else f"fma({self.c(b2)}, lnT, {a2})"
+        inner = f"fma({self.c(-t2)}, invT, pyro::vconst({a2}))"
+        return inner if b2 == 0 else f"fma({self.c(b2)}, lnT, {inner})"
+
+    def ec(self, x: float) -> str:
+        """A constant factor in an exponent, in the current base."""
+        if self.base2:
+            x = float(_DEC.divide(decimal.Decimal(x), _LN2))
+        return self.c(x)
 
     # --- thermo ---------------------------------------------------------
     def _flags(self, w: _Writer, T: str = "T"):
@@ -364,13 +418,13 @@ class _Lowering:
             return expr
         hi, lo = coeffs(sp.high), coeffs(sp.low)
         if hi == lo:
-            w(f"E[{k}] = {self.fexp}({poly(hi)});  // {sp.name}")
+            w(f"E[{k}] = {self.gexp}({poly(hi)});  // {sp.name}")
         else:
             # both ranges evaluated and pinned so the choice stays a
             # per-lane select rather than a divergent branch
             w(f"{{ double gh = {poly(hi)}, gl = {poly(lo)};")
             w('  asm volatile("" : "+v"(gh), "+v"(gl));')
-            w(f"  E[{k}] = {self.fexp}({self.tmid_flag[sp.t_mid]} ? gh : gl);"
+            w(f"  E[{k}] = {self.gexp}({self.tmid_flag[sp.t_mid]} ? gh : gl);"
               f" }}  // {sp.name}")
 
     def kinv_expr(self, r: Reaction) -> str:
@@ -416,43 +470,63 @@ class _Lowering:
             w(f'asm volatile("" : {ops});')
 
     # --- kinetics -------------------------------------------------------
-    def arrhenius(self, rate) -> str:
+    def arrhenius_parts(self, rate) -> Tuple[str, Optional[str]]:
+        """(factor, exponent) of A T^b exp(-Ta/T): a power law with a small
+        integer b is a factor without exponent, anything else an exponent
+        (in the current base) without factor, or with the factor A when
+        Ta = 0."""
         a, b, ta = rate.A, rate.b, rate.t_a
         c = self.c
         if ta == 0:
             if b == 0:
-                return c(a)
+                return c(a), None
             if _is_small_int(b):
                 if b < 0:
-                    return f"({c(a)} * pyro::ipow<{int(-b)}>(invT))"
-                return f"({c(a)} * pyro::ipow<{int(b)}>(T))"
-            return f"({c(a)} * {self.fexp}({c(b)} * lnT))"
-        lna = math.log(a)
-        if b == 0:
-            return f"{self.fexp}(fma({c(-ta)}, invT, {c(lna)}))"
-        return (f"{self.fexp}(fma({c(b)}, lnT, fma({c(-ta)}, invT, "
-                f"{c(lna)})))")
+                    return f"({c(a)} * pyro::ipow<{int(-b)}>(invT))", None
+                return f"({c(a)} * pyro::ipow<{int(b)}>(T))", None
+            if not self.base2:
+                return c(a), f"{c(b)} * lnT"
+        return "", self.exponent(b, ta, _DEC.ln(decimal.Decimal(a))
+                                 if self.base2 else math.log(a))
 
-    def rate_ratio(self, lo, hi) -> str:
-        """k_lo / k_hi as one expression: a constant times an integer power
-        of T when both are pure power laws, else one exp of the difference
-        of the Arrhenius exponents."""
+    def arrhenius(self, rate) -> str:
+        fac, ex = self.arrhenius_parts(rate)
+        if ex is None:
+            return fac
+        e = f"{self.fexp}({ex})"
+        return f"({fac} * {e})" if fac else e
+
+    def rate_ratio_parts(self, lo, hi) -> Tuple[str, Optional[str]]:
+        """k_lo / k_hi: a constant times an integer power of T (a factor)
+        when both are pure power laws, else the difference of the Arrhenius
+        exponents (an exponent)."""
         db = lo.b - hi.b
         if lo.t_a == 0 and hi.t_a == 0 and _is_small_int(db):
             c = self.c(lo.A / hi.A)
             if db == 0:
-                return c
+                return c, None
             if db < 0:
-                return f"({c} * pyro::ipow<{int(-db)}>(invT))"
-            return f"({c} * pyro::ipow<{int(db)}>(T))"
-        dlna = math.log(lo.A) - math.log(hi.A)
-        dta = lo.t_a - hi.t_a
-        return (f"{self.fexp}(fma({self.c(db)}, lnT, fma({self.c(-dta)}, "
-                f"invT, {self.c(dlna)})))")
+                return f"({c} * pyro::ipow<{int(-db)}>(invT))", None
+            return f"({c} * pyro::ipow<{int(db)}>(T))", None
+        D = decimal.Decimal
+        dlna = (_DEC.ln(D(lo.A)) - _DEC.ln(D(hi.A)) if self.base2
+                else math.log(lo.A) - math.log(hi.A))
+        return "", self.exponent(db, lo.t_a - hi.t_a, dlna)
+
+    def rate_ratio(self, lo, hi) -> str:
+        fac, ex = self.rate_ratio_parts(lo, hi)
+        return fac if ex is None else f"{self.fexp}({ex})"
+
+    @staticmethod
+    def body_key(r: Reaction):
+        """Reactions with equal keys have the same [M]."""
+        return (r.default_efficiency, tuple(sorted(r.efficiencies)))
 
     def third_body(self, r: Reaction, C: str = "C", Ctot: str = "Ctot") -> str:
         """[M] = d Ctot + sum_k (eff_k - d) C_k (chem_expr.py:327-345); with
         ``C``/``Ctot`` naming tangent arrays it gives the tangent of [M]."""
+        if C == "C" and self.body_key(r) in self.m_shared:
+            return self.m_shared[self.body_key(r)][0]
         d = r.default_efficiency
         terms = []
         for sp, eff in r.efficiencies:
@@ -478,7 +552,9 @@ class _Lowering:
     def kf_block(self, w: _Writer, r: Reaction, out: str = "kf"):
         """Emit statements defining ``out`` = forward rate coefficient with
         falloff and three-body factors (codegen/python.py:398-473)."""
-        if r.kind == "falloff":
+        if r.kind == "falloff" and self.base2:
+            self._kf_falloff_base2(w, r, out)
+        elif r.kind == "falloff":
             w(f"const double khi = {self.arrhenius(r.high_rate)};")
             w(f"const double pr = ({self.third_body(r)}) * "
               f"{self.rate_ratio(r.low_rate, r.high_rate)};")
@@ -504,6 +580,52 @@ class _Lowering:
             w(f"const double {out} = {self.arrhenius(r.rate)} * ({self.third_body(r)});")
         else:
             w(f"const double {out} = {self.arrhenius(r.rate)};")
+
+    def _kf_falloff_base2(self, w: _Writer, r: Reaction, out: str):
+        """Falloff k_f with every exponent in base 2.  Troe's
+        F = 10^(Fc/(1 + f1^2)) = 2^(f2/(1 + f1^2)) with f2 = log2 of the
+        centre and f1 formed of base-2 logarithms (numerator and denominator
+        both divided by log10 2, which leaves f1); log2 P_r is log2 [M] plus
+        the exponent of k_lo/k_hi, and k_inf's exponent is added to F's, so
+        that one power serves both."""
+        c = self.c
+        fh, eh = self.arrhenius_parts(r.high_rate)
+        fr, er = self.rate_ratio_parts(r.low_rate, r.high_rate)
+        key = self.body_key(r)
+        if key in self.m_shared:
+            M, lM = self.m_shared[key]
+        else:
+            w(f"const double M = {self.third_body(r)};")
+            M, lM = "M", "pyro::log2p(M)"
+        if er is None:
+            w(f"const double pr = {M} * {fr};")
+        else:
+            w(f"const double er = {er};")
+            w(f"const double pr = {M} * pyro::exp2p(er);")
+        if r.falloff_type != "Troe":
+            k = self.arrhenius(r.high_rate)
+            w(f"const double {out} = {k} * (pr * pyro::recip(1.0 + pr));")
+            return
+        tp = r.troe
+        t1 = f"{c(1.0 - tp[0])} * pyro::exp2p(T * {self.ec(-1.0 / tp[1])})"
+        t2 = f"{c(tp[0])} * pyro::exp2p(T * {self.ec(-1.0 / tp[2])})"
+        s = f"{t1} + {t2}"
+        if len(tp) == 4:
+            s += f" + pyro::exp2p({self.ec(-tp[3])} * invT)"
+        w(f"const double fc = pyro::log2p({s});")
+        lpr = "pyro::log2p(pr)" if er is None else f"{lM} + er"
+        w(f"const double lpr = {lpr};")
+        w(f"const double u = lpr + fma(-0.67, fc, {c(-0.4 / LOG10_2)});")
+        w(f"const double nn = fma(-1.27, fc, {c(0.75 / LOG10_2)});")
+        w("const double f1 = pr > 0.0 ? u * pyro::recip(fma(-0.14, u, nn)) "
+          f": {lit(-1 / 0.14)};")
+        w("const double rF = pyro::recip(fma(f1, f1, 1.0));")
+        if eh is None:
+            w("const double kF = pyro::exp2p(fc * rF);")
+        else:
+            w(f"const double kF = pyro::exp2p(fma(fc, rF, {eh}));")
+        w(f"const double {out} = {fh + ' * ' if fh else ''}"
+          "(kF * pr * pyro::recip(1.0 + pr));")
 
     # --- derivatives (forward mode, hand-written per reaction kind) ---------
     def dlnk(self, rate) -> str:
@@ -843,7 +965,8 @@ def species_uses(L: _Lowering, r: Reaction):
         c |= {L.idx[sp] for sp, _ in r.products}
         if L.species_kc:
             e = {L.idx[sp] for sp, _ in list(r.reactants) + list(r.products)}
-    if r.kind in ("three-body", "falloff"):
+    if r.kind in ("three-body", "falloff") and \
+            L.body_key(r) not in L.m_shared:
         c |= {k for k, _ in L.efficiency_terms(r)}
     return c, e, w
 
@@ -954,15 +1077,31 @@ def _emit_wdot_lazy(w: _Writer, L: _Lowering):
     w.ind += 1
     if L.tuning.get("recip1", True):
         L.frecip = "pyro::recip1"
-    if L.tuning.get("ctable", True):
+    if L.tuning.get("wdot_ctable", False):
         L.tab = []
         w("pyro::cptr K = (pyro::cptr)kTabWdotLazy;")
         w('asm volatile("" : "+s"(K));')
-    w("const double lnT = log(T);")
-    w("const double invT = 1.0 / T;")
+    if L.tuning.get("base2", True):
+        L.base2, L.fexp, L.gexp = True, "pyro::exp2p", "pyro::expp"
+        w("const double lnT = pyro::finite_or_huge(log(T));")
+        w("const double invT = pyro::finite_or_huge(1.0 / T);")
+        # third-body sums [M] of several reactions (GRI-3.0: one sum serves
+        # 26 reactions, another 6) are formed with the total concentration
+        # and kept, with their base-2 logarithms, beside the mass fractions
+        # in LDS
+        bodies = [L.body_key(r) for r in m.reactions
+                  if r.kind in ("three-body", "falloff")]
+        if L.uses_ctot() and L.tuning.get("ystash", 0) > 8:
+            shared = [k for k in sorted(set(bodies), key=bodies.index)
+                      if bodies.count(k) >= 3][:4]
+            L.m_shared = {k: None for k in shared}
+    else:
+        w("const double lnT = log(T);")
+        w("const double invT = 1.0 / T;")
     if rev:
         L.emit_gibbs_prologue(w)
-    order = reaction_order(L, L.tuning.get("order_tries", 8))
+    zform = rev and L.tuning.get("zform", False)
+    order = reaction_order(L, L.tuning.get("wdot_tries", 8))
     uses = [species_uses(L, r) for r in m.reactions]
     # ystash: the mass fractions of that many species, the last to open,
     # kept in LDS by the total-concentration pass for their opening (one
@@ -972,10 +1111,13 @@ def _emit_wdot_lazy(w: _Writer, L: _Lowering):
         for k in uses[ri][0]:
             first_use.setdefault(k, pos)
     nst = int(L.tuning.get("ystash", 0)) if L.uses_ctot() else 0
+    if L.m_shared:
+        nst = min(nst, L.ns, 40 - 2 * len(L.m_shared))
     stash = {k: n for n, k in enumerate(sorted(
         first_use, key=lambda k: -first_use[k])[:nst])}
     if stash:
-        w(f"__shared__ double ys[{len(stash)}][kWdotBlock];")
+        w(f"__shared__ double ys[{len(stash) + 2 * len(L.m_shared)}]"
+          "[kWdotBlock];")
         w("double* ysw = &ys[0][threadIdx.x];")
     if L.uses_ctot():
         # the total concentration needs every species up front; the values
@@ -987,13 +1129,26 @@ def _emit_wdot_lazy(w: _Writer, L: _Lowering):
             w("#pragma unroll")
             w("for (int k = 0; k < NS; ++k) "
               "Ctot += kInvW[k] * rho * Y[k * ldY + i];")
+        eff = {key: {L.idx[sp]: e - key[0] for sp, e in key[1]}
+               for key in L.m_shared}
+        for j in range(len(eff)):
+            w(f"double M{j} = 0.0;")
         for k in range(L.ns) if stash else ():
+            w(f"{{ const double y = Y[{k} * ldY + i], "
+              f"c = kInvW[{k}] * rho * y; Ctot += c;")
+            for j, e in enumerate(eff.values()):
+                if e.get(k, 0.0) != 0.0:
+                    w(f"  M{j} = fma({lit(e[k])}, c, M{j});")
             if k in stash:
-                w(f"{{ const double y = Y[{k} * ldY + i]; "
-                  f"Ctot += kInvW[{k}] * rho * y; "
-                  f"ysw[{stash[k]} * kWdotBlock] = y; }}")
-            else:
-                w(f"Ctot += kInvW[{k}] * rho * Y[{k} * ldY + i];")
+                w(f"  ysw[{stash[k]} * kWdotBlock] = y;")
+            w("}")
+        for j, key in enumerate(eff):
+            a = len(stash) + 2 * j
+            w(f"M{j} = fma({lit(key[0])}, Ctot, M{j});")
+            w(f"ysw[{a} * kWdotBlock] = M{j};")
+            w(f"ysw[{a + 1} * kWdotBlock] = pyro::log2p(M{j});")
+            L.m_shared[key] = (f"ysr[{a} * kWdotBlock]",
+                               f"ysr[{a + 1} * kWdotBlock]")
     if stash:
         w("pyro::lptr ysr = (pyro::lptr)ysw;")
     # Yg: Y as a global-memory pointer that is passed through an empty asm
@@ -1006,7 +1161,6 @@ def _emit_wdot_lazy(w: _Writer, L: _Lowering):
     #   q = k_f prod_r F_r (prod_r Z_r - (RT/p0)^dnu prod_p Z_p)
     # (= k_f (prod_r C_r - K_c^-1 prod_p C_p)): one reciprocal per species
     # instead of one per reaction
-    zform = rev and L.tuning.get("zform", False)
     if zform:
         w("double F[NS], Z[NS];")
     last_w = {}
@@ -1098,6 +1252,7 @@ def _emit_wdot_lazy(w: _Writer, L: _Lowering):
                 + ", ".join(lit(x) for x in tab) + "};")
         w.lines.insert(table_at, decl)
         L.tab = None
+    L.base2, L.fexp, L.gexp, L.m_shared = False, "exp", "exp", {}
 
 
 def _emit_wdot_jac(w: _Writer, L: _Lowering):

@@ -100,4 +100,95 @@ __device__ __forceinline__ double recip(double x) {
   return fma(r, e, r);
 }
 
+// A uniform constant copied to vector registers by one v_mov_b64: an FMA
+// takes one scalar operand, and of two constants the compiler copies the
+// second with two v_mov_b32.
+__device__ __forceinline__ double vconst(double c) {
+  double v;
+  asm("v_mov_b64 %0, %1" : "=v"(v) : "s"(c));
+  return v;
+}
+
+// 2^y for the exponents of rate coefficients, which are formed in base 2
+// from constants scaled by log2(e): n = rint(y), then the degree-11
+// polynomial through 2^f at Chebyshev nodes on |f| <= 1/2 (2e-17 relative),
+// f = y - n exact.  15 VALU operations against about 25 for exp (no
+// argument reduction by ln 2 and no range selects: v_cvt_i32_f64 saturates
+// and v_ldexp_f64 gives 0 and infinity by itself).  NaN gives NaN; y must
+// not be infinite (finite_or_huge bounds what it is formed of).
+__device__ __forceinline__ double exp2p(double y) {
+  const double n = __builtin_rint(y);
+  const double f = y - n;
+  double p = fma(4.4558179083360645e-10, f, vconst(7.074194297288521e-09));
+  p = fma(p, f, 1.0178057087733941e-07);
+  p = fma(p, f, 1.3215432535912375e-06);
+  p = fma(p, f, 1.5252733841556773e-05);
+  p = fma(p, f, 0.00015403530463724353);
+  p = fma(p, f, 0.001333355814640647);
+  p = fma(p, f, 0.009618129107587256);
+  p = fma(p, f, 0.055504108664821625);
+  p = fma(p, f, 0.24022650695910158);
+  p = fma(p, f, 0.6931471805599453);
+  p = fma(p, f, 1.0);
+  return __builtin_amdgcn_ldexp(p, static_cast<int>(n));
+}
+
+// e^x likewise, for exponents whose coefficients are the mechanism's own
+// decimals (the Gibbs functions: scaled to base 2 their seven rounded terms
+// would cost accuracy): r = x - n ln 2 in two parts, then the degree-11
+// polynomial through e^r at Chebyshev nodes on |r| <= ln 2 / 2 (2e-17).
+__device__ __forceinline__ double expp(double x) {
+  const double n = __builtin_rint(x * 1.4426950408889634);
+  double r = fma(n, -0.6931471805599453, x);
+  r = fma(n, -2.3190468138462996e-17, r);
+  double p = fma(2.5110037605963777e-08, r, vconst(2.763263963904103e-07));
+  p = fma(p, r, 2.755724091857897e-06);
+  p = fma(p, r, 2.4801485482328494e-05);
+  p = fma(p, r, 0.00019841269890047113);
+  p = fma(p, r, 0.0013888888952314775);
+  p = fma(p, r, 0.008333333333319601);
+  p = fma(p, r, 0.0416666666664881);
+  p = fma(p, r, 0.1666666666666668);
+  p = fma(p, r, 0.5000000000000019);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  return __builtin_amdgcn_ldexp(p, static_cast<int>(n));
+}
+
+// log2(x) of a positive x to about 2^-52 of max(1, |log2 x|): x = m 2^e with
+// m in [sqrt(1/2), sqrt 2), s = (m - 1)/(m + 1), log2 m = s P(s^2) with P
+// the degree-7 polynomial through its Chebyshev nodes (2e-17 relative).
+// NaN for x <= 0.  The Troe terms need only its absolute error.
+__device__ __forceinline__ double log2p(double x) {
+  double m = __builtin_amdgcn_frexp_mant(x);
+  int e = __builtin_amdgcn_frexp_exp(x);
+  const bool lo = m < 0.70710678118654752;
+  m = lo ? m + m : m;
+  e = lo ? e - 1 : e;
+  const double d = m + 1.0;
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(r, fma(-d, r, 1.0), r);
+  const double nu = m - 1.0;
+  double s = nu * r;
+  s = fma(r, fma(-d, s, nu), s);
+  const double z = s * s;
+  double p = 0.2136589569431927;
+  p = fma(p, z, 0.2209130842311768);
+  p = fma(p, z, 0.262334352504183);
+  p = fma(p, z, 0.32059853491395984);
+  p = fma(p, z, 0.4121985858409005);
+  p = fma(p, z, 0.5770780163455203);
+  p = fma(p, z, 0.9617966939259898);
+  p = fma(p, z, 2.8853900817779268);
+  const double v = fma(s, p, static_cast<double>(e));
+  return x > 0.0 ? v : __builtin_nan("");
+}
+
+// x with infinities replaced by a huge finite value of their sign, so that
+// an exponent formed of it saturates instead of meeting inf - inf in exp2p
+// (1/T and ln T at T = 0 or infinite, once per cell).
+__device__ __forceinline__ double finite_or_huge(double x) {
+  return __builtin_fabs(x) == __builtin_inf() ? __builtin_copysign(1e290, x) : x;
+}
+
 }  // namespace pyro
