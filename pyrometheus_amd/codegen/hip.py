@@ -179,23 +179,19 @@ class _Writer:
 #:           GRI-3.0 cells, timed side by side);
 #:  nt_rq -- the same for the per-reaction outputs (k_f and the like: no
 #:           change measured, off).
-#:  base2 -- the lazy omega-dot pass takes the powers of its exponents with
-#:           pyro::exp2p / expp (15 and 17 VALU operations) instead of exp
-#:           (about 25), writes Troe's blending in base-2 logarithms (one log2
-#:           per reaction beside one per shared [M], k_inf's power merged
-#:           with F's) and forms [M] sums that several reactions share once
-#:           per cell: 19,910 -> 12,965 VALU operations per wave;
-#:  wdot_ctable -- that pass reads its constants from one table through
-#:           scalar loads instead of literals.  Off: each reaction waits for
+#:  wdot_ctable -- the omega-dot passes read their constants from one table
+#:           through scalar loads instead of literals.  Off: each reaction waits for
 #:           its loads, which a full chip hides and a partly filled one does
 #:           not (16,384 GRI-3.0 cells 56 against 40 us, 131,072 cells 88
 #:           against 69 us, 2^22 cells 2.02 against 2.00 ms);
 #: (GRI-3.0, 2^24 cells: 16.6 ms with the species arrays held in registers,
-#: 12.1 ms lazy at two waves per SIMD, 11.35 ms with zform, 7.8 ms with
-#: base2.  What bounds it there is FP64 issue at the clock that the card
+#: 12.1 ms lazy at two waves per SIMD, 11.35 ms with zform, 8.2 ms with the
+#: powers of pyro::exp2p / expp (15 and 17 VALU operations, against about 25
+#: of exp), Troe's blending in base-2 logarithms and shared [M] sums: 19,910
+#: -> 12,965 VALU operations per wave.  What bounds it there is FP64 issue at the clock that the card
 #: holds under it: an independent FP64 operation takes 2.2 ns per SIMD with
 #: every SIMD busy, 13k of them 1.8 of the 2.0 ms of 2^22 cells.)
-DEFAULT_TUNING = {"pin": True, "pin_every": 3, "kc": "species", "ctable": True,
+DEFAULT_TUNING = {"pin": True, "pin_every": 3, "kc": "species",
                   "lazy": True, "wdot_waves": 2, "deriv_waves": 0,
                   "lazy_fence": 1, "order_tries": 8, "wdot_tries": 21, "prefetch": 4,
                   "zform": True, "jac_groups": 4, "ystash": 39}
@@ -256,14 +252,8 @@ class _Lowering:
         self.tab = None  # list of tabulated constants while emitting a table
         # value -> index into tab, when constants are shared while emitting
         self.tab_index = None
-        # the power taken of the Arrhenius and of the Gibbs exponents
-        self.fexp = "exp"
-        self.gexp = "exp"
         # reciprocal in K_c^-1 (products of Gibbs factors)
         self.frecip = "pyro::recip"
-        # Arrhenius and Gibbs exponents in base 2 (constants scaled by
-        # log2(e)) and their powers from pyro::exp2p
-        self.base2 = False
         # efficiency key -> ([M], log2 [M]) variables, formed once per cell
         self.m_shared = {}
         # K_c^-1 from E[] of the products and F[] = 1 / E[] of the
@@ -289,17 +279,13 @@ class _Lowering:
         return f"K[{len(self.tab) - 1}]"
 
     def exponent(self, b: float, ta: float, ln_a) -> str:
-        """b ln T - Ta/T + ln A in the current base, each constant rounded
-        once.  In base 2 the constants b log2(e) and Ta log2(e) are no
-        longer the mechanism's own decimals; what their rounding leaves at
+        """(b ln T - Ta/T + ln A) log2(e), the exponent pyro::exp2p takes,
+        each constant rounded once.  The constants b log2(e) and Ta log2(e)
+        are not the mechanism's own decimals; what their rounding leaves at
         1200 K is put into the third, which keeps the exponent's error at
         that of the base-e form (GRI-3.0 over 300..2500 K: 2.4e-15 rms
         against 2.5e-15; 2.6e-15 without)."""
         D = decimal.Decimal
-        if not self.base2:
-            inner = (self.c(float(ln_a)) if ta == 0 else
-                     f"fma({self.c(-ta)}, invT, {self.c(float(ln_a))})")
-            return inner if b == 0 else f"fma({self.c(b)}, lnT, {inner})"
         t0 = D(1200)
         bx, tx, ax = (_DEC.divide(x, _LN2) for x in (D(b), D(ta), ln_a))
         b2, t2 = float(bx), float(tx)
@@ -311,10 +297,15 @@ class _Lowering:
         return inner if b2 == 0 else f"fma({self.c(b2)}, lnT, {inner})"
 
     def ec(self, x: float) -> str:
-        """A constant factor in an exponent, in the current base."""
-        if self.base2:
-            x = float(_DEC.divide(decimal.Decimal(x), _LN2))
-        return self.c(x)
+        """A constant factor of an exponent in base 2."""
+        return self.c(float(_DEC.divide(decimal.Decimal(x), _LN2)))
+
+    def shared_bodies(self) -> List[Tuple]:
+        """Keys of the third-body sums of three or more reactions."""
+        keys = [self.body_key(r) for r in self.m.reactions
+                if r.kind in ("three-body", "falloff")]
+        return [k for k in sorted(set(keys), key=keys.index)
+                if keys.count(k) >= 3][:4]
 
     # --- thermo ---------------------------------------------------------
     def _flags(self, w: _Writer, T: str = "T"):
@@ -418,13 +409,13 @@ class _Lowering:
             return expr
         hi, lo = coeffs(sp.high), coeffs(sp.low)
         if hi == lo:
-            w(f"E[{k}] = {self.gexp}({poly(hi)});  // {sp.name}")
+            w(f"E[{k}] = pyro::expp({poly(hi)});  // {sp.name}")
         else:
             # both ranges evaluated and pinned so the choice stays a
             # per-lane select rather than a divergent branch
             w(f"{{ double gh = {poly(hi)}, gl = {poly(lo)};")
             w('  asm volatile("" : "+v"(gh), "+v"(gl));')
-            w(f"  E[{k}] = {self.gexp}({self.tmid_flag[sp.t_mid]} ? gh : gl);"
+            w(f"  E[{k}] = pyro::expp({self.tmid_flag[sp.t_mid]} ? gh : gl);"
               f" }}  // {sp.name}")
 
     def kinv_expr(self, r: Reaction) -> str:
@@ -448,10 +439,10 @@ class _Lowering:
         return (f"({side(r.products, num_extra)}) * "
                 f"{self.frecip}({side(r.reactants, den_extra)})")
 
-    def zform_terms(self, r: Reaction) -> str:
-        """prod_r F_r * (prod_r Z_r - (RT/p0)^dnu prod_p Z_p), the rate of
-        progress over k_f of a reversible reaction (balanced, integer nu)
-        from the per-species F_k = exp(-g'_k), Z_k = C_k exp(g'_k)."""
+    def zform_parts(self, r: Reaction) -> Tuple[str, str, str]:
+        """prod_r F_r, prod_r Z_r and (RT/p0)^dnu prod_p Z_p of a reversible
+        reaction (balanced, integer nu), from the per-species
+        F_k = exp(-g'_k) and Z_k = C_k exp(g'_k)."""
         def side(d, arr, extra=()):
             ts = []
             for sp, nu in d:
@@ -461,8 +452,14 @@ class _Lowering:
         dnu = int(sum(nu for _, nu in r.products)
                   - sum(nu for _, nu in r.reactants))
         ex = ["rtp"] * dnu if dnu > 0 else ["prt"] * (-dnu)
-        return (f"({side(r.reactants, 'F')}) * ({side(r.reactants, 'Z')} - "
-                f"{side(r.products, 'Z', ex)})")
+        return (side(r.reactants, 'F'), side(r.reactants, 'Z'),
+                side(r.products, 'Z', ex))
+
+    def zform_terms(self, r: Reaction) -> str:
+        """The rate of progress over k_f of a reversible reaction:
+        prod_r F_r * (prod_r Z_r - (RT/p0)^dnu prod_p Z_p)."""
+        fac, fwd, bwd = self.zform_parts(r)
+        return f"({fac}) * ({fwd} - {bwd})"
 
     def pin(self, w: _Writer, names: List[str]):
         if self.tuning["pin"] and names:
@@ -471,10 +468,9 @@ class _Lowering:
 
     # --- kinetics -------------------------------------------------------
     def arrhenius_parts(self, rate) -> Tuple[str, Optional[str]]:
-        """(factor, exponent) of A T^b exp(-Ta/T): a power law with a small
-        integer b is a factor without exponent, anything else an exponent
-        (in the current base) without factor, or with the factor A when
-        Ta = 0."""
+        """(factor, exponent in base 2) of A T^b exp(-Ta/T): a power law
+        with a small integer b is a factor without exponent, anything else
+        an exponent without factor."""
         a, b, ta = rate.A, rate.b, rate.t_a
         c = self.c
         if ta == 0:
@@ -484,17 +480,11 @@ class _Lowering:
                 if b < 0:
                     return f"({c(a)} * pyro::ipow<{int(-b)}>(invT))", None
                 return f"({c(a)} * pyro::ipow<{int(b)}>(T))", None
-            if not self.base2:
-                return c(a), f"{c(b)} * lnT"
-        return "", self.exponent(b, ta, _DEC.ln(decimal.Decimal(a))
-                                 if self.base2 else math.log(a))
+        return "", self.exponent(b, ta, _DEC.ln(decimal.Decimal(a)))
 
     def arrhenius(self, rate) -> str:
         fac, ex = self.arrhenius_parts(rate)
-        if ex is None:
-            return fac
-        e = f"{self.fexp}({ex})"
-        return f"({fac} * {e})" if fac else e
+        return fac if ex is None else f"pyro::exp2p({ex})"
 
     def rate_ratio_parts(self, lo, hi) -> Tuple[str, Optional[str]]:
         """k_lo / k_hi: a constant times an integer power of T (a factor)
@@ -509,13 +499,12 @@ class _Lowering:
                 return f"({c} * pyro::ipow<{int(-db)}>(invT))", None
             return f"({c} * pyro::ipow<{int(db)}>(T))", None
         D = decimal.Decimal
-        dlna = (_DEC.ln(D(lo.A)) - _DEC.ln(D(hi.A)) if self.base2
-                else math.log(lo.A) - math.log(hi.A))
-        return "", self.exponent(db, lo.t_a - hi.t_a, dlna)
+        return "", self.exponent(db, lo.t_a - hi.t_a,
+                                 _DEC.ln(D(lo.A)) - _DEC.ln(D(hi.A)))
 
     def rate_ratio(self, lo, hi) -> str:
         fac, ex = self.rate_ratio_parts(lo, hi)
-        return fac if ex is None else f"{self.fexp}({ex})"
+        return fac if ex is None else f"pyro::exp2p({ex})"
 
     @staticmethod
     def body_key(r: Reaction):
@@ -552,36 +541,14 @@ class _Lowering:
     def kf_block(self, w: _Writer, r: Reaction, out: str = "kf"):
         """Emit statements defining ``out`` = forward rate coefficient with
         falloff and three-body factors (codegen/python.py:398-473)."""
-        if r.kind == "falloff" and self.base2:
-            self._kf_falloff_base2(w, r, out)
-        elif r.kind == "falloff":
-            w(f"const double khi = {self.arrhenius(r.high_rate)};")
-            w(f"const double pr = ({self.third_body(r)}) * "
-              f"{self.rate_ratio(r.low_rate, r.high_rate)};")
-            if r.falloff_type == "Troe":
-                tp = r.troe
-                c = self.c
-                t1 = f"({c(1.0 - tp[0])} * exp(T * {c(-1.0 / tp[1])}))"
-                t2 = f"({c(tp[0])} * exp(T * {c(-1.0 / tp[2])}))"
-                s = f"{t1} + {t2}"
-                if len(tp) == 4:
-                    s += f" + exp({c(-tp[3])} * invT)"
-                w(f"const double fc = log10({s});")
-                w("const double lpr = log10(pr);")
-                w("const double cc = fma(-0.67, fc, -0.4);")
-                w("const double nn = fma(-1.27, fc, 0.75);")
-                w("const double f1 = pr > 0.0 ? (lpr + cc) * pyro::recip("
-                  f"fma(-0.14, lpr + cc, nn)) : {lit(-1 / 0.14)};")
-                w("const double fF = exp10(fc * pyro::recip(fma(f1, f1, 1.0)));")
-                w(f"const double {out} = khi * (fF * pr * pyro::recip(1.0 + pr));")
-            else:
-                w(f"const double {out} = khi * (pr * pyro::recip(1.0 + pr));")
+        if r.kind == "falloff":
+            self._kf_falloff(w, r, out)
         elif r.kind == "three-body":
             w(f"const double {out} = {self.arrhenius(r.rate)} * ({self.third_body(r)});")
         else:
             w(f"const double {out} = {self.arrhenius(r.rate)};")
 
-    def _kf_falloff_base2(self, w: _Writer, r: Reaction, out: str):
+    def _kf_falloff(self, w: _Writer, r: Reaction, out: str):
         """Falloff k_f with every exponent in base 2.  Troe's
         F = 10^(Fc/(1 + f1^2)) = 2^(f2/(1 + f1^2)) with f2 = log2 of the
         centre and f1 formed of base-2 logarithms (numerator and denominator
@@ -640,51 +607,61 @@ class _Lowering:
         dkfM = dkf/d[M] (chem_expr.py:310-421 differentiated by hand)."""
         c = self.c
         if r.kind == "falloff":
-            ln10 = math.log(10.0)
-            w(f"const double khi = {self.arrhenius(r.high_rate)};")
+            ln2 = math.log(2.0)
+            fh, eh = self.arrhenius_parts(r.high_rate)
+            fr, er = self.rate_ratio_parts(r.low_rate, r.high_rate)
             w(f"const double ahi = {self.dlnk(r.high_rate)};")
             w(f"const double alo = {self.dlnk(r.low_rate)};")
-            w(f"const double ratio = {self.rate_ratio(r.low_rate, r.high_rate)};")
+            if er is None:
+                w(f"const double ratio = {fr};")
+            else:
+                w(f"const double er = {er};")
+                w("const double ratio = pyro::exp2p(er);")
             w(f"const double M = {self.third_body(r)};")
             w("const double pr = M * ratio;")
             w("const double rpr1 = pyro::recip(1.0 + pr);")
             if r.falloff_type == "Troe":
+                # base-2 logarithms and powers as in _kf_falloff
                 tp = r.troe
-                w(f"const double e1 = exp(T * {c(-1.0 / tp[1])});")
-                w(f"const double e2 = exp(T * {c(-1.0 / tp[2])});")
+                w(f"const double e1 = pyro::exp2p(T * {self.ec(-1.0 / tp[1])});")
+                w(f"const double e2 = pyro::exp2p(T * {self.ec(-1.0 / tp[2])});")
                 S = f"fma({c(1.0 - tp[0])}, e1, {c(tp[0])} * e2)"
                 dS = (f"fma({c((1.0 - tp[0]) * (-1.0 / tp[1]))}, e1, "
                       f"{c(tp[0] * (-1.0 / tp[2]))} * e2)")
                 if len(tp) == 4:
-                    w(f"const double e3 = exp({c(-tp[3])} * invT);")
+                    w(f"const double e3 = pyro::exp2p({self.ec(-tp[3])} * invT);")
                     S = f"({S} + e3)"
                     dS = f"fma({c(tp[3])} * invT * invT, e3, {dS})"
                 w(f"const double sS = {S};")
-                w(f"const double fc = log10(sS);")
-                w(f"const double dfc = {dS} * pyro::recip(sS) * {c(1 / ln10)};")
-                w("const double lpr = log10(pr);")
-                w("const double cc = fma(-0.67, fc, -0.4);")
-                w("const double nn = fma(-1.27, fc, 0.75);")
-                w("const double u = lpr + cc;")
+                w(f"const double fc = pyro::log2p(sS);")
+                w(f"const double dfc = {dS} * pyro::recip(sS) * {c(1 / ln2)};")
+                w("const double lpr = " + ("pyro::log2p(pr);" if er is None
+                                           else "pyro::log2p(M) + er;"))
+                w(f"const double u = lpr + fma(-0.67, fc, {c(-0.4 / LOG10_2)});")
+                w(f"const double nn = fma(-1.27, fc, {c(0.75 / LOG10_2)});")
                 w("const double rden = pyro::recip(fma(-0.14, u, nn));")
                 w("const bool pos = pr > 0.0;")
                 w(f"const double f1 = pos ? u * rden : {lit(-1 / 0.14)};")
                 w("const double ropf = pyro::recip(fma(f1, f1, 1.0));")
-                w("const double fF = exp10(fc * ropf);")
+                # k_inf F: F's power merged with k_inf's
+                kF = ("fc * ropf" if eh is None else f"fma(fc, ropf, {eh})")
+                w(f"const double kF = {fh + ' * ' if fh else ''}"
+                  f"pyro::exp2p({kF});")
                 w("const double dlF_df1 = -2.0 * fc * f1 * ropf * ropf;")
                 w("const double df1_du = pos ? nn * rden * rden : 0.0;")
                 w("const double df1_dn = pos ? -u * rden * rden : 0.0;")
                 w("const double dlF_dL = dlF_df1 * df1_du;")
                 w("const double dlF_dfc = fma(dlF_df1, fma(-0.67, df1_du, "
                   "-1.27 * df1_dn), ropf);")
-                w(f"const double dlF_dT = fma(dlF_dL * {c(1 / ln10)}, alo - ahi, "
+                w(f"const double dlF_dT = fma(dlF_dL * {c(1 / ln2)}, alo - ahi, "
                   "dlF_dfc * dfc);")
-                w("const double kf = khi * (fF * pr * rpr1);")
-                w("const double dkfM = khi * fF * ratio * fma(dlF_dL, rpr1, "
+                w("const double kf = kF * pr * rpr1;")
+                w("const double dkfM = kF * ratio * fma(dlF_dL, rpr1, "
                   "rpr1 * rpr1);")
-                w(f"const double dkfT = kf * (ahi + fma({c(ln10)}, dlF_dT, "
+                w(f"const double dkfT = kf * (ahi + fma({c(ln2)}, dlF_dT, "
                   "(alo - ahi) * rpr1));")
             else:
+                w(f"const double khi = {self.arrhenius(r.high_rate)};")
                 w("const double kf = khi * (pr * rpr1);")
                 w("const double dkfM = khi * ratio * rpr1 * rpr1;")
                 w("const double dkfT = kf * fma(alo - ahi, rpr1, ahi);")
@@ -883,13 +860,18 @@ def _emit_thermo(w: _Writer, L: _Lowering):
     w("")
 
 
+def _emit_lnT(w: _Writer, T: str = "T", suffix: str = ""):
+    """ln T and 1/T as the exponents read them (finite, for exp2p)."""
+    w(f"const double lnT{suffix} = pyro::finite_or_huge(log({T}));")
+    w(f"const double invT{suffix} = pyro::finite_or_huge(1.0 / {T});")
+
+
 def _kin_prologue(w: _Writer, L: _Lowering, need_g: bool):
-    w("const double lnT = log(T);")
-    w("const double invT = 1.0 / T;")
+    _emit_lnT(w)
     if need_g:
         w("const double c0 = log(kOneAtm / (kGasConstant * T));")
         w("double g[NS];")
-        w("species_g_rt(T, lnT, invT, g);")
+        w("species_g_rt(T, log(T), 1.0 / T, g);")
     if L.uses_ctot():
         w("double Ctot = 0.0;")
         w("#pragma unroll")
@@ -903,7 +885,7 @@ def _emit_wdot(w: _Writer, L: _Lowering):
     w("__device__ __forceinline__ void net_production_rates(const double T, "
       "const double (&C)[NS], double (&w)[NS]) {")
     w.ind += 1
-    if L.tuning.get("ctable", True):
+    if L.tuning.get("wdot_ctable", False):
         L.tab = []
         # constants are read from a table in constant memory through a
         # pointer the optimiser cannot see through: uniform scalar loads
@@ -927,7 +909,7 @@ def _emit_wdot(w: _Writer, L: _Lowering):
         rf = L.prod_expr(L.reactant_pairs(r))
         if r.reversible:
             rr = L.prod_expr([(L.idx[sp], nu) for sp, nu in r.products])
-            kinv = L.kinv_expr(r) if L.species_kc else f"exp({L.nlk_expr(r)})"
+            kinv = L.kinv_expr(r) if L.species_kc else f"pyro::expp({L.nlk_expr(r)})"
             w(f"const double q = kf * ({rf} - {kinv} * {rr});")
         else:
             w(f"const double q = kf * ({rf});")
@@ -1081,23 +1063,13 @@ def _emit_wdot_lazy(w: _Writer, L: _Lowering):
         L.tab = []
         w("pyro::cptr K = (pyro::cptr)kTabWdotLazy;")
         w('asm volatile("" : "+s"(K));')
-    if L.tuning.get("base2", True):
-        L.base2, L.fexp, L.gexp = True, "pyro::exp2p", "pyro::expp"
-        w("const double lnT = pyro::finite_or_huge(log(T));")
-        w("const double invT = pyro::finite_or_huge(1.0 / T);")
-        # third-body sums [M] of several reactions (GRI-3.0: one sum serves
-        # 26 reactions, another 6) are formed with the total concentration
-        # and kept, with their base-2 logarithms, beside the mass fractions
-        # in LDS
-        bodies = [L.body_key(r) for r in m.reactions
-                  if r.kind in ("three-body", "falloff")]
-        if L.uses_ctot() and L.tuning.get("ystash", 0) > 8:
-            shared = [k for k in sorted(set(bodies), key=bodies.index)
-                      if bodies.count(k) >= 3][:4]
-            L.m_shared = {k: None for k in shared}
-    else:
-        w("const double lnT = log(T);")
-        w("const double invT = 1.0 / T;")
+    _emit_lnT(w)
+    # third-body sums [M] of several reactions (GRI-3.0: one sum serves
+    # 26 reactions, another 6) are formed with the total concentration
+    # and kept, with their base-2 logarithms, beside the mass fractions
+    # in LDS
+    if L.uses_ctot() and L.tuning.get("ystash", 0) > 8:
+        L.m_shared = {k: None for k in L.shared_bodies()}
     if rev:
         L.emit_gibbs_prologue(w)
     zform = rev and L.tuning.get("zform", False)
@@ -1252,7 +1224,7 @@ def _emit_wdot_lazy(w: _Writer, L: _Lowering):
                 + ", ".join(lit(x) for x in tab) + "};")
         w.lines.insert(table_at, decl)
         L.tab = None
-    L.base2, L.fexp, L.gexp, L.m_shared = False, "exp", "exp", {}
+    L.m_shared = {}
 
 
 def _emit_wdot_jac(w: _Writer, L: _Lowering):
@@ -1293,7 +1265,7 @@ def _emit_wdot_jac(w: _Writer, L: _Lowering):
             ppairs = [(L.idx[sp], nu) for sp, nu in r.products]
             w(f"const double pb = {L.prod_expr(ppairs)};")
             dpb = dict(L.prod_partials(ppairs))
-            kinv = L.kinv_expr(r) if L.species_kc else f"exp({L.nlk_expr(r)})"
+            kinv = L.kinv_expr(r) if L.species_kc else f"pyro::expp({L.nlk_expr(r)})"
             w(f"const double kinv = {kinv};")
             dnu = sum(nu for _, nu in r.products) - sum(nu for _, nu in r.reactants)
             hs = [f"{lit(-nu)} * hrt[{L.idx[sp]}]" for sp, nu in r.products]
@@ -1356,7 +1328,7 @@ def _reverse_parts(w: _Writer, L: _Lowering, r: Reaction):
         ppairs = [(L.idx[sp], nu) for sp, nu in r.products]
         w(f"const double pb = {L.prod_expr(ppairs)};")
         dpb = dict(L.prod_partials(ppairs))
-        kinv = L.kinv_expr(r) if L.species_kc else f"exp({L.nlk_expr(r)})"
+        kinv = L.kinv_expr(r) if L.species_kc else f"pyro::expp({L.nlk_expr(r)})"
         w(f"const double kinv = {kinv};")
         dnu = sum(nu for _, nu in r.products) - sum(nu for _, nu in r.reactants)
         hs = [f"{lit(-nu)} * hrt[{L.idx[sp]}]" for sp, nu in r.products]
@@ -1475,8 +1447,7 @@ def _emit_wdot_jvp_lazy(w: _Writer, L: _Lowering):
         return
     w(sig)
     w.ind += 1
-    w("const double lnT = log(T);")
-    w("const double invT = 1.0 / T;")
+    _emit_lnT(w)
     if rev:
         L.emit_gibbs_prologue(w)
     w("const double sv = vY ? rho : 0.0;")
@@ -1666,8 +1637,7 @@ def _emit_wdot_vjp_lazy(w: _Writer, L: _Lowering):
         return
     w(sig)
     w.ind += 1
-    w("const double lnT = log(T);")
-    w("const double invT = 1.0 / T;")
+    _emit_lnT(w)
     if rev:
         L.emit_gibbs_prologue(w)
     w("pyro::gptr Yg = (pyro::gptr)Y;")
@@ -2113,8 +2083,7 @@ def _emit_jac_fused_gibbs(w: _Writer, L: _Lowering, gibbs: bool):
     w.ind += 1
     if gibbs:
         w("constexpr int hs = kJacFusedCells;")
-        w("const double lnT = log(T);")
-        w("const double invT = 1.0 / T;")
+        _emit_lnT(w)
         L.emit_gibbs_prologue(w)
         basis = ["omlnT", "T", "T2", "T3", "T4", "invT"]
         for k, sp in enumerate(L.m.species):
@@ -2136,8 +2105,8 @@ def _emit_jac_fused_gibbs(w: _Writer, L: _Lowering, gibbs: bool):
                 w(f"double gh = {poly(hi)}, gl = {poly(lo)};")
                 w('asm volatile("" : "+v"(gh), "+v"(gl));')
                 w(f"const double g = {L.tmid_flag[sp.t_mid]} ? gh : gl;")
-            w(f"Et[{k} * hs] = exp(g);")
-            w(f"Ft[{k} * hs] = exp(-g);")
+            w(f"Et[{k} * hs] = pyro::expp(g);")
+            w(f"Ft[{k} * hs] = pyro::expp(-g);")
             w.ind -= 1
             w("}")
     w.ind -= 1
@@ -2211,8 +2180,8 @@ def _emit_source_jacobian_fused(w: _Writer, L: _Lowering):
     w("const double dT00 = 1.0 / cp;")
     w("const double dr00 = -rT0 * dT00;")
     w("const double rm0 = -rho * mmw;  // drho_m = -rT dT_m + rm / W_m")
-    w("const double lnT0 = log(T0);")
-    w("const double invT0 = 1.0 / T0;")
+    w("const double lnT0 = pyro::finite_or_huge(log(T0));")
+    w("const double invT0 = pyro::finite_or_huge(1.0 / T0);")
     w("const double omlnT0 = 1.0 - lnT0;")
     w("const double T20 = T0 * T0, T30 = T20 * T0, T40 = T30 * T0;")
     w("const double rkT0 = -cp * invT0 * (1.0 / kGasConstant);")
@@ -2386,7 +2355,7 @@ def _emit_source_jacobian_fused(w: _Writer, L: _Lowering):
                 L.kinv_f = False
             else:
                 _emit_kinv_linear(w, L, r, "lk")
-                w("const double kinv = exp(lk);")
+                w("const double kinv = pyro::expp(lk);")
             # sum over reactants minus products of nu h/RT, from the dT table
             net: Dict[int, float] = {}
             for sp, n2 in r.reactants:
@@ -2533,8 +2502,8 @@ def _emit_reaction_quantities(w: _Writer, L: _Lowering):
             w("if ((MASK & 1) && okf) " + st("okf", idx, "kf"))
             w("if ((MASK & 2) && onlk) " + st("onlk", idx, "nlk"))
             w("if ((MASK & 4) && orf) " + st("orf", idx, "kf * pf"))
-            w("if ((MASK & 8) && orr) " + st("orr", idx, "kf * exp(nlk) * pb"))
-            w("if ((MASK & 16) && onet) " + st("onet", idx, "kf * (pf - exp(nlk) * pb)"))
+            w("if ((MASK & 8) && orr) " + st("orr", idx, "kf * pyro::expp(nlk) * pb"))
+            w("if ((MASK & 16) && onet) " + st("onet", idx, "kf * (pf - pyro::expp(nlk) * pb)"))
         else:
             w(f"const double pf = {rf};")
             w("if ((MASK & 1) && okf) " + st("okf", idx, "kf"))
@@ -2547,6 +2516,120 @@ def _emit_reaction_quantities(w: _Writer, L: _Lowering):
     w.ind -= 1
     w("}")
     w("")
+
+
+def gibbs_range(L: _Lowering, bound: float = 600.0) -> Tuple[float, float]:
+    """The temperatures around 1000 K over which |sum nu_k g'_k| of either
+    side of every reversible reaction, and each |g'_k|, is at most
+    ``bound``, so that products of Gibbs factors neither overflow nor
+    underflow."""
+    m = L.m
+
+    def fits(T):
+        g = []
+        for k, sp in enumerate(m.species):
+            c = sp.high if T > sp.t_mid else sp.low
+            g.append(c[0] * (1 - math.log(T)) - c[1] / 2 * T
+                     - c[2] / 6 * T ** 2 - c[3] / 12 * T ** 3
+                     - c[4] / 20 * T ** 4 + (c[5] - L.shift_m[k]) / T
+                     - c[6] - L.shift_n[k])
+        sides = [abs(sum(nu * g[L.idx[s]] for s, nu in side))
+                 for r in m.reactions if r.reversible
+                 for side in (r.reactants, r.products)]
+        return max(max(map(abs, g)), max(sides, default=0.0)) <= bound
+    lo = hi = 1000
+    while lo > 20 and fits(lo - 1):
+        lo -= 1
+    while hi < 10000 and fits(hi + 50):
+        hi += 50
+    return float(lo), float(hi)
+
+
+def _emit_progress_lazy(w: _Writer, L: _Lowering):
+    """Reverse (MASK 8) or net (MASK 16) rates of progress alone, with the
+    species opened along a reaction order as in ``_emit_wdot_lazy`` and K_c^-1
+    as products of the per-species F and Z of ``zform_terms``: 53 powers for
+    GRI-3.0 where the general form takes one per reversible reaction (309)
+    and holds every species' C and g."""
+    m = L.m
+    rev = any(r.reversible for r in m.reactions)
+    w(f"constexpr bool kProgressLazy = "
+      f"{'true' if rev and L.species_kc else 'false'};")
+    tmin, tmax = gibbs_range(L)
+    w(f"constexpr double kProgressTmin = {lit(tmin)};")
+    w(f"constexpr double kProgressTmax = {lit(tmax)};")
+    w("template <int MASK>")
+    w("__device__ __forceinline__ void progress_lazy(const double T, "
+      "const double* __restrict__ Cin, const int64_t ldC, const int64_t i, "
+      "const int64_t ld, double* __restrict__ out) {")
+    w.ind += 1
+    if not (rev and L.species_kc):
+        w.ind -= 1
+        w("}")
+        w("")
+        return
+    w("pyro::gptr Cg = (pyro::gptr)Cin;")
+    _emit_lnT(w)
+    L.emit_gibbs_prologue(w)
+    if L.uses_ctot():
+        L.m_shared = {k: (f"M{j}", f"lM{j}")
+                      for j, k in enumerate(L.shared_bodies())}
+        eff = {key: {L.idx[sp]: e - key[0] for sp, e in key[1]}
+               for key in L.m_shared}
+        w("double Ctot = 0.0;")
+        for j in range(len(eff)):
+            w(f"double M{j} = 0.0;")
+        for k in range(L.ns):
+            w(f"{{ const double c = Cg[{k} * ldC + i]; Ctot += c;")
+            for j, e in enumerate(eff.values()):
+                if e.get(k, 0.0) != 0.0:
+                    w(f"  M{j} = fma({lit(e[k])}, c, M{j});")
+            w("}")
+        for j, key in enumerate(eff):
+            w(f"M{j} = fma({lit(key[0])}, Ctot, M{j});")
+            w(f"const double lM{j} = pyro::log2p(M{j});")
+    uses = []
+    for r in m.reactions:
+        c, e, _ = species_uses(L, r)
+        uses.append((c, e, set()))
+    order = reaction_order(L, L.tuning.get("wdot_tries", 8), uses)
+    w("double C[NS], E[NS], F[NS], Z[NS];")
+    open_c, open_e = set(), set()
+    for pos, ri in enumerate(order):
+        r = m.reactions[ri]
+        c_u, e_u, _ = uses[ri]
+        if c_u - open_c:
+            w('asm volatile("" : "+s"(Cg));')
+        for k in sorted(c_u - open_c):
+            w(f"C[{k}] = Cg[{k} * ldC + i];")
+        for k in sorted(e_u - open_e):
+            L.emit_gibbs_one(w, k)
+            w(f"F[{k}] = pyro::recip(E[{k}]);")
+            w(f"Z[{k}] = C[{k}] * E[{k}];")
+        open_c |= c_u
+        open_e |= e_u
+        w(f"{{  // R{ri}: {r.equation} [{r.reaction_type}]")
+        w.ind += 1
+        if r.reversible:
+            L.kf_block(w, r)
+            fac, fwd, bwd = L.zform_parts(r)
+            w(f"out[{ri} * ld + i] = MASK == 8 ? kf * (({fac}) * ({bwd})) "
+              f": kf * (({fac}) * ({fwd} - {bwd}));")
+        else:
+            w("if (MASK == 8) {")
+            w(f"  out[{ri} * ld + i] = 0.0;")
+            w("} else {")
+            L.kf_block(w, r)
+            w(f"out[{ri} * ld + i] = "
+              f"kf * ({L.prod_expr(L.reactant_pairs(r))});")
+            w("}")
+        w.ind -= 1
+        w("}")
+        w('asm volatile("" ::: "memory");')
+    w.ind -= 1
+    w("}")
+    w("")
+    L.m_shared = {}
 
 
 def _emit_creation_destruction(w: _Writer, L: _Lowering):
@@ -2565,7 +2648,7 @@ def _emit_creation_destruction(w: _Writer, L: _Lowering):
         w(f"const double qf = kf * ({L.prod_expr(L.reactant_pairs(r))});")
         if r.reversible:
             rr = L.prod_expr([(L.idx[sp], nu) for sp, nu in r.products])
-            w(f"const double qr = kf * exp({L.nlk_expr(r)}) * ({rr});")
+            w(f"const double qr = kf * pyro::expp({L.nlk_expr(r)}) * ({rr});")
         for sp, nu in r.reactants:
             k = L.idx[sp]
             w(f"dd[{k}] = fma({lit(nu)}, qf, dd[{k}]);")
@@ -2611,8 +2694,7 @@ def _emit_creation_destruction_lazy(w: _Writer, L: _Lowering):
         w("")
         return
     rev = any(r.reversible for r in m.reactions)
-    w("const double lnT = log(T);")
-    w("const double invT = 1.0 / T;")
+    _emit_lnT(w)
     if rev:
         w("const double c0 = log(kOneAtm / (kGasConstant * T));")
         L._flags(w)
@@ -2661,7 +2743,7 @@ def _emit_creation_destruction_lazy(w: _Writer, L: _Lowering):
         w(f"const double qf = kf * ({L.prod_expr(L.reactant_pairs(r))});")
         if r.reversible:
             rr = L.prod_expr([(L.idx[sp], nu) for sp, nu in r.products])
-            w(f"const double qr = kf * exp({L.nlk_expr(r)}) * ({rr});")
+            w(f"const double qr = kf * pyro::expp({L.nlk_expr(r)}) * ({rr});")
         for sp, nu in r.reactants:
             k = L.idx[sp]
             w(f"dd[{k}] = fma({lit(nu)}, qf, dd[{k}]);")
@@ -2727,6 +2809,7 @@ class HipCodeGenerator(CodeGenerator):
         _emit_wdot(w, L)
         _emit_wdot_lazy(w, L)
         _emit_reaction_quantities(w, L)
+        _emit_progress_lazy(w, L)
         _emit_creation_destruction(w, L)
         _emit_creation_destruction_lazy(w, L)
         _emit_wdot_jvp(w, L)
