@@ -33,46 +33,168 @@ namespace pyro_spike {
 
 using pyro_bt::bcast;
 
-// Gauss-Jordan as pyro_bt::gauss_jordan_dpp for four independent systems
-// per wave, one per 16-lane row: lanes base..base+NV-1 (base = 16 g) hold
-// the rows of system g, gl = lane - base.  The pivot of each row of lanes
-// comes from its own DPP max-reduction; the pivot row's entries are read
-// with ds_bpermute from lane base + p, p differing between the systems.
-template <int NV, int W>
-__device__ __forceinline__ void gauss_jordan_grp(double (&a)[W], int lane,
-                                                 int& my_k, bool& singular) {
+// ---- rows within 16-lane groups (NV <= 16) --------------------------------
+// Lane gl of a 16-lane group holds logical row gl, so the pivot row of step
+// k is always lane k and its entries reach the other lanes through DPP
+// (row_newbcast:k reads lane k of each 16-lane row): one v_fmac_f64_dpp
+// updates a column, 4 to 5 cycles each and no LDS.  (Pivot rows left in
+// place, differing between the groups, take two ds_bpermute_b32 per entry,
+// 6 cycles of the compute unit's one LDS pipe each: about 510 per block row
+// at NV = 10, which bound the sweep -- 523 us for the 143k rows of 256
+// flamelets, where the FMAs need about 60.)
+// A DPP operand must have been written two wait states before; the compiler
+// does not see into the asm blocks, so each begins with s_nop 1.
+
+// lane K's v in every lane of its 16-lane row
+template <int K>
+__device__ __forceinline__ double row_bcast(double v) {
+  double o;
+  asm("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+      : "=v"(o) : "v"(v), "n"(K));
+  return o;
+}
+
+#define PYRO_FMB(D, S) \
+  "\n\tv_fmac_f64_dpp " D ", " S ", %[m] row_newbcast:%[k] row_mask:0xf bank_mask:0xf"
+// acc[j] += (lane K's src[j]) m for j in [0, N), arrays distinct
+template <int K, int N>
+__device__ __forceinline__ void fmac_bcast(double* acc, const double* src,
+                                           double m) {
+  if constexpr (N >= 8) {
+    asm("s_nop 1" PYRO_FMB("%0", "%8") PYRO_FMB("%1", "%9")
+        PYRO_FMB("%2", "%10") PYRO_FMB("%3", "%11") PYRO_FMB("%4", "%12")
+        PYRO_FMB("%5", "%13") PYRO_FMB("%6", "%14") PYRO_FMB("%7", "%15")
+        : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]),
+          "+&v"(acc[4]), "+&v"(acc[5]), "+&v"(acc[6]), "+&v"(acc[7])
+        : "v"(src[0]), "v"(src[1]), "v"(src[2]), "v"(src[3]), "v"(src[4]),
+          "v"(src[5]), "v"(src[6]), "v"(src[7]), [m] "v"(m), [k] "n"(K));
+    fmac_bcast<K, N - 8>(acc + 8, src + 8, m);
+  } else if constexpr (N >= 2) {
+    asm("s_nop 1" PYRO_FMB("%0", "%2") PYRO_FMB("%1", "%3")
+        : "+&v"(acc[0]), "+&v"(acc[1])
+        : "v"(src[0]), "v"(src[1]), [m] "v"(m), [k] "n"(K));
+    fmac_bcast<K, N - 2>(acc + 2, src + 2, m);
+  } else if constexpr (N == 1) {
+    asm("s_nop 1" PYRO_FMB("%0", "%1")
+        : "+&v"(acc[0]) : "v"(src[0]), [m] "v"(m), [k] "n"(K));
+  }
+}
+// a[j] += (lane K's a[j]) m for j in [0, N)
+template <int K, int N>
+__device__ __forceinline__ void fmac_bcast_self(double* a, double m) {
+  if constexpr (N >= 8) {
+    asm("s_nop 1" PYRO_FMB("%0", "%0") PYRO_FMB("%1", "%1")
+        PYRO_FMB("%2", "%2") PYRO_FMB("%3", "%3") PYRO_FMB("%4", "%4")
+        PYRO_FMB("%5", "%5") PYRO_FMB("%6", "%6") PYRO_FMB("%7", "%7")
+        : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]),
+          "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7])
+        : [m] "v"(m), [k] "n"(K));
+    fmac_bcast_self<K, N - 8>(a + 8, m);
+  } else if constexpr (N >= 4) {
+    asm("s_nop 1" PYRO_FMB("%0", "%0") PYRO_FMB("%1", "%1")
+        PYRO_FMB("%2", "%2") PYRO_FMB("%3", "%3")
+        : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
+        : [m] "v"(m), [k] "n"(K));
+    fmac_bcast_self<K, N - 4>(a + 4, m);
+  } else if constexpr (N >= 1) {
+    asm("s_nop 1" PYRO_FMB("%0", "%0")
+        : "+&v"(a[0]) : [m] "v"(m), [k] "n"(K));
+    fmac_bcast_self<K, N - 1>(a + 1, m);
+  }
+}
+// a += (lane K's x) m, b += (lane K's y) n
+template <int K>
+__device__ __forceinline__ void fmac_bcast_2(double& a, double x, double m,
+                                             double& b, double y, double n) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %2, %4 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf"
+      : "+&v"(a), "+&v"(b) : "v"(x), "v"(y), "v"(m), "v"(n), "n"(K));
+}
+#undef PYRO_FMB
+
+// Gauss-Jordan on the rows [A | ...] of the wave's four 16-lane groups, each
+// an independent system; on return lane gl holds row gl of [I | X].  Rows
+// are scaled so that their largest |A| entry is 1; the pivot of column K is
+// row K unless another unused row's entry is over kPivotRatio times larger
+// in some group, which then exchanges that group's row K with its largest
+// (threshold partial pivoting: against the strict form, on the blocks of
+// sandiego flamelets from time steps of 1e-8 s to steady, the same or a
+// smaller error of the solution, with 0.0 to 0.3 exchanges per block row
+// instead of 0 to 3).  kSlot: columns NV..2NV-1 start as a diagonal, so
+// that, while no rows have been exchanged, only the first K+1 of them are
+// live at step K.
+constexpr double kPivotRatio = 10.0;
+
+// Orders this wave's LDS accesses for the compiler (the hardware executes a
+// wave's LDS instructions in order; wave-local data needs no barrier).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int NV, int W, bool kSlot, int K>
+__device__ __forceinline__ void gj_row16_step(double (&a)[W], int gl,
+                                              double (*rows)[2][W], bool& full,
+                                              bool& singular) {
+  double piv = row_bcast<K>(a[K]);
+  double inv = pyro::recip(piv);
+  if constexpr (K + 1 < NV) {
+    const bool worse = gl > K && gl < NV &&
+                       fabs(a[K]) > kPivotRatio * fabs(piv);
+    if (__builtin_amdgcn_ballot_w64(worse) != 0ull) {
+      // exchange row K with the largest candidate where one is much larger:
+      // those two lanes of the group pass their rows through LDS
+      const int lane = threadIdx.x & 63;
+      const unsigned best = pyro_bt::row16_max_u32(
+          pyro_bt::pivot_key(a[K], gl >= K && gl < NV, lane));
+      const unsigned any = pyro_bt::row16_max_u32(worse ? 1u : 0u);
+      const int p = 63 - static_cast<int>(best & 63u) - (lane & 48);
+      if (any && best >= 64u && (gl == K || gl == p)) {
+        double(&mine)[W] = rows[lane >> 4][gl == K ? 0 : 1];
+        double(&other)[W] = rows[lane >> 4][gl == K ? 1 : 0];
+#pragma unroll
+        for (int j = K; j < W; ++j) mine[j] = a[j];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = K; j < W; ++j) a[j] = other[j];
+      }
+      wave_lds_fence();
+      full = true;
+      piv = row_bcast<K>(a[K]);
+      inv = pyro::recip(piv);
+    }
+  }
+  singular = singular || !(fabs(piv) > 0.0);
+  const double g = (gl == K) ? inv - 1.0 : -(a[K] * inv);
+  fmac_bcast_self<K, NV - 1 - K>(a + K + 1, g);
+  if constexpr (kSlot) {
+    fmac_bcast_self<K, K + 1>(a + NV, g);
+    fmac_bcast_self<K, W - 2 * NV>(a + 2 * NV, g);
+    if constexpr (K + 1 < NV) {
+      if (full) fmac_bcast_self<K, NV - 1 - K>(a + NV + K + 1, g);
+    }
+  } else {
+    fmac_bcast_self<K, W - NV>(a + NV, g);
+  }
+  if constexpr (K + 1 < NV)
+    gj_row16_step<NV, W, kSlot, K + 1>(a, gl, rows, full, singular);
+}
+
+template <int NV, int W, bool kSlot>
+__device__ __forceinline__ void gauss_jordan_row16(double (&a)[W], int gl,
+                                                   double (*rows)[2][W],
+                                                   bool& singular) {
   static_assert(NV <= 16, "one 16-lane row holds the rows");
-  const int base = lane & 48;
-  const int gl = lane - base;
-  const bool active = gl < NV;
-  {
-    double mx = 0.0;
+  double mx = 0.0;
 #pragma unroll
-    for (int c = 0; c < NV; ++c) mx = fmax(mx, fabs(a[c]));
-    const double sc = mx > 0.0 ? pyro::recip(mx) : 1.0;
+  for (int c = 0; c < NV; ++c) mx = fmax(mx, fabs(a[c]));
+  const double sc = mx > 0.0 ? pyro::recip(mx) : 1.0;
 #pragma unroll
-    for (int c = 0; c < W; ++c) a[c] *= sc;
-  }
-  unsigned used = 0u;
-  constexpr unsigned all = (1u << NV) - 1u;
-  my_k = -1;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    // every lane of the 16-lane row holds the row's maximum key
-    const unsigned best = pyro_bt::row16_max_u32(
-        pyro_bt::pivot_key(a[k], active && !((used >> gl) & 1u), lane));
-    const int p = best >= 64u ? 63 - static_cast<int>(best & 63u) - base
-                              : __builtin_ctz(~used & all);
-    used |= 1u << p;
-    const int src = base + p;
-    const double piv = __shfl(a[k], src);
-    singular = singular || !(fabs(piv) > 0.0);
-    const double inv = pyro::recip(piv);
-    const double g = (gl == p) ? 1.0 - inv : a[k] * inv;
-#pragma unroll
-    for (int j = k + 1; j < W; ++j) a[j] = fma(-g, __shfl(a[j], src), a[j]);
-    if (gl == p) my_k = k;
-  }
+  for (int c = 0; c < W; ++c) a[c] *= sc;
+  bool full = !kSlot;
+  gj_row16_step<NV, W, kSlot, 0>(a, gl, rows, full, singular);
 }
 
 // The partition sweeps for NV <= 16, four sweeps per wave: sweep task
@@ -92,6 +214,7 @@ k_spike_sweep_grp(const double* __restrict__ L, const double* __restrict__ C,
                   int* __restrict__ n_singular) {
   constexpr int W = 3 * NV + 1;
   constexpr int MW = 2 * NV + 1;
+  __shared__ double rows[4][2][W];
   const int lane = threadIdx.x;
   const int gl = lane & 15;
   const int64_t task = static_cast<int64_t>(blockIdx.x) * 4 + (lane >> 4);
@@ -114,9 +237,7 @@ k_spike_sweep_grp(const double* __restrict__ L, const double* __restrict__ C,
   auto back_coef = [&](int64_t i) -> double {
     return down ? L[i] : U[i - 1];
   };
-  const int base = lane & 48;
   double a[W];
-  int my_k = gl;
   {
     const int64_t i = row(0);
 #pragma unroll
@@ -142,27 +263,24 @@ k_spike_sweep_grp(const double* __restrict__ L, const double* __restrict__ C,
       bpre = back_coef(i);
       spre = slot_coef(i1);
     }
-    gauss_jordan_grp<NV, W>(a, lane, my_k, singular);
+    gauss_jordan_row16<NV, W, true>(a, gl, rows, singular);
     if (down && active) {
-      double* f = fact + (i * NV + my_k) * MW;
+      double* f = fact + (i * NV + gl) * MW;
 #pragma unroll
       for (int c = 0; c < MW; ++c) f[c] = a[NV + c];
     }
     if (t + 1 == m) break;
-    const int k = active ? my_k : 0;
-    const int src = base + k;
     const double l = bpre;
 #pragma unroll
-    for (int c = 0; c < NV; ++c)
-      a[c] = fma(-l, a[NV + c], __shfl(cpre[c], src));
-    a[2 * NV] = fma(-l, a[2 * NV], __shfl(rpre, src));
+    for (int c = 0; c < NV; ++c) a[c] = fma(-l, a[NV + c], cpre[c]);
+    a[2 * NV] = fma(-l, a[2 * NV], rpre);
 #pragma unroll
     for (int c = 0; c < NV; ++c) a[2 * NV + 1 + c] *= -l;
 #pragma unroll
-    for (int c = 0; c < NV; ++c) a[NV + c] = (c == k) ? spre : 0.0;
+    for (int c = 0; c < NV; ++c) a[NV + c] = (c == r) ? spre : 0.0;
   }
   if (active) {
-    double* mp = maps + ((part * 2 + (down ? 0 : 1)) * NV + my_k) * MW;
+    double* mp = maps + ((part * 2 + (down ? 0 : 1)) * NV + gl) * MW;
     mp[0] = a[2 * NV];
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
@@ -186,6 +304,27 @@ k_spike_sweep_grp(const double* __restrict__ L, const double* __restrict__ C,
 //   t_q = tau_q + H_q t_{q+1}.  Z_j of the interface between q and q+1
 //   receives (b_q, t_{q+1}).  red holds per partition and row
 //   [beta | G row | tau | H row] (2 NV + 2 doubles).
+// The rows sit in 16-lane groups as in the sweep (all four groups of the
+// wave do the same work), so every product term and every elimination step
+// is one v_fmac_f64_dpp.
+template <int NV, int M>
+__device__ __forceinline__ void mul_add_row16(double (&acc)[NV + 1],
+                                              const double (&x)[NV + 1],
+                                              const double (&b)[NV]) {
+  // acc += b X, X's row M in lane M of the group
+  fmac_bcast<M, NV + 1>(acc, x, b[M]);
+  if constexpr (M + 1 < NV) mul_add_row16<NV, M + 1>(acc, x, b);
+}
+
+// (bt[0], bt[1]) += (g . t, h . t), t's entry M in lane M of the group
+template <int NV, int M>
+__device__ __forceinline__ void dot_row16(double (&bt)[2], double t,
+                                          const double (&g)[NV],
+                                          const double (&h)[NV]) {
+  fmac_bcast_2<M>(bt[0], t, g[M], bt[1], t, h[M]);
+  if constexpr (M + 1 < NV) dot_row16<NV, M + 1>(bt, t, g, h);
+}
+
 template <int NV>
 __global__ void __launch_bounds__(64)
 k_spike_reduced(const double* __restrict__ maps,
@@ -195,10 +334,12 @@ k_spike_reduced(const double* __restrict__ maps,
   constexpr int N2 = 2 * NV;
   constexpr int RW = 2 * NV + 2;
   constexpr int WA = 2 * NV + 1;
+  __shared__ double rows[4][2][WA];
   const int sy = blockIdx.x;
   const int lane = threadIdx.x;
-  const bool active = lane < NV;
-  const int r = active ? lane : 0;
+  const int gl = lane & 15;
+  const bool writer = lane < NV;
+  const int r = gl < NV ? gl : 0;
   const int64_t j0 = roff[sy], j1 = roff[sy + 1];
   const int64_t nq = j1 - j0 + 1;   // partitions of this system
   if (nq < 2) return;
@@ -207,101 +348,110 @@ k_spike_reduced(const double* __restrict__ maps,
   auto mrow = [&](int64_t q, int dir) {
     return maps + ((q * 2 + dir) * NV + r) * MW;
   };
-  auto rrow = [&](int64_t q, int row) { return red + (q * NV + row) * RW; };
+  auto rrow = [&](int64_t q) { return red + (q * NV + r) * RW; };
   bool singular = false;
-  double beta, G[NV];
-  {
-    const double* md = mrow(q0, 0);
-    beta = md[0];
+  double G[NV + 1];  // row r of [G | beta]
+  auto load = [&](int64_t q, int dir, double (&o)[MW]) {
+    const double* m = mrow(q, dir);
 #pragma unroll
-    for (int c = 0; c < NV; ++c) G[c] = md[1 + NV + c];
-    if (active) {
-      double* o = rrow(q0, r);
-      o[0] = beta;
+    for (int c = 0; c < MW; ++c) o[c] = m[c];
+  };
+  auto store_G = [&](int64_t q) {
+    if (!writer) return;
+    double* o = rrow(q);
+    o[0] = G[NV];
 #pragma unroll
-      for (int c = 0; c < NV; ++c) o[1 + c] = G[c];
-    }
-  }
+    for (int c = 0; c < NV; ++c) o[1 + c] = G[c];
+  };
+  double mu[MW], md[MW];
+  load(q0, 0, md);
+#pragma unroll
+  for (int c = 0; c < NV; ++c) G[c] = md[1 + NV + c];
+  G[NV] = md[0];
+  store_G(q0);
+  load(q0 + 1, 1, mu);
+  load(q0 + 1, 0, md);
   for (int64_t q = q0 + 1; q < q0 + nq; ++q) {
-    const double* mu = mrow(q, 1);
-    const double* md = mrow(q, 0);
-    // [I - B' G | a' + B' beta | D'] in row r
+    // the next partition's maps, in flight during this one
+    double mun[MW], mdn[MW];
+    const int64_t qn = q + 1 < q0 + nq ? q + 1 : q;
+    load(qn, 1, mun);
+    load(qn, 0, mdn);
+    // [I - B' G | a' + B' beta | D'] in row r, and [P | a + B beta],
+    // P = B G_{q-1}, before G is replaced
+    double b[NV], Q[NV + 1], P[NV + 1], H[NV + 1];
+#pragma unroll
+    for (int c = 0; c < NV; ++c) {
+      b[c] = mu[1 + c];
+      Q[c] = P[c] = 0.0;
+    }
+    Q[NV] = mu[0];
+    P[NV] = md[0];
+    mul_add_row16<NV, 0>(Q, G, b);
+#pragma unroll
+    for (int c = 0; c < NV; ++c) b[c] = md[1 + c];
+    mul_add_row16<NV, 0>(P, G, b);
     double aug[WA];
 #pragma unroll
-    for (int c = 0; c < NV; ++c) aug[c] = (c == r) ? 1.0 : 0.0;
-    double rhs = mu[0];
-#pragma unroll
-    for (int mm = 0; mm < NV; ++mm) {
-      const double bp = mu[1 + mm];
-      rhs = fma(bp, pyro_bt::bcast(beta, mm), rhs);
-#pragma unroll
-      for (int c = 0; c < NV; ++c)
-        aug[c] = fma(-bp, pyro_bt::bcast(G[c], mm), aug[c]);
+    for (int c = 0; c < NV; ++c) {
+      aug[c] = ((c == r) ? 1.0 : 0.0) - Q[c];
+      aug[NV + 1 + c] = mu[1 + NV + c];
     }
-    aug[NV] = rhs;
+    aug[NV] = Q[NV];
+    gauss_jordan_row16<NV, WA, false>(aug, gl, rows, singular);
+    // row r of [H | tau]
 #pragma unroll
-    for (int c = 0; c < NV; ++c) aug[NV + 1 + c] = mu[1 + NV + c];
-    // P = B G_{q-1} (row r) before G is replaced
-    double P[NV], bsum = md[0];
+    for (int c = 0; c < NV; ++c) H[c] = aug[NV + 1 + c];
+    H[NV] = aug[NV];
+    if (writer) {
+      double* o = rrow(q);
+      o[1 + NV] = H[NV];
 #pragma unroll
-    for (int c = 0; c < NV; ++c) P[c] = 0.0;
-#pragma unroll
-    for (int mm = 0; mm < NV; ++mm) {
-      const double bm = md[1 + mm];
-      bsum = fma(bm, pyro_bt::bcast(beta, mm), bsum);
-#pragma unroll
-      for (int c = 0; c < NV; ++c)
-        P[c] = fma(bm, pyro_bt::bcast(G[c], mm), P[c]);
+      for (int c = 0; c < NV; ++c) o[2 + NV + c] = H[c];
     }
-    int my_k, perm[NV];
-    pyro_bt::gauss_jordan_dpp<NV, WA>(aug, lane, my_k, perm, singular);
-    // lane perm[m] holds row m of [tau | H]
-    if (active) {
-      double* o = rrow(q, my_k);
-      o[1 + NV] = aug[NV];
+    // [G | beta]_q = [D | a + B beta] + P [H | tau]
 #pragma unroll
-      for (int c = 0; c < NV; ++c) o[2 + NV + c] = aug[NV + 1 + c];
+    for (int c = 0; c < NV; ++c) {
+      b[c] = P[c];
+      G[c] = md[1 + NV + c];
     }
-    // G_{q-1} is no longer needed: G_q = D + P H accumulates in place
+    G[NV] = P[NV];
+    mul_add_row16<NV, 0>(G, H, b);
+    store_G(q);
 #pragma unroll
-    for (int c = 0; c < NV; ++c) G[c] = md[1 + NV + c];
-#pragma unroll
-    for (int mm = 0; mm < NV; ++mm) {
-      const int src = perm[mm];
-      const double pm = P[mm];
-      bsum = fma(pm, pyro_bt::bcast(aug[NV], src), bsum);
-#pragma unroll
-      for (int c = 0; c < NV; ++c)
-        G[c] = fma(pm, pyro_bt::bcast(aug[NV + 1 + c], src), G[c]);
-    }
-    beta = bsum;
-    if (active) {
-      double* o = rrow(q, r);
-      o[0] = beta;
-#pragma unroll
-      for (int c = 0; c < NV; ++c) o[1 + c] = G[c];
+    for (int c = 0; c < MW; ++c) {
+      mu[c] = mun[c];
+      md[c] = mdn[c];
     }
   }
-  // back substitution; t in natural row order, lane r holds t[r]
+  // back substitution; t in natural row order, lane r holds t[r].  A lane
+  // reads only rows of red that it (or its twin in the first group) wrote.
+  __syncthreads();
   const int64_t ql = q0 + nq - 1;
-  double t = rrow(ql, r)[1 + NV];
-  for (int64_t q = ql - 1; q >= q0; --q) {
-    const double* o = rrow(q, r);
-    double b = o[0];
+  double t = rrow(ql)[1 + NV];
+  double o[RW];
+  auto load_red = [&](int64_t q) {
+    const double* p = rrow(q);
 #pragma unroll
-    for (int mm = 0; mm < NV; ++mm) b = fma(o[1 + mm], pyro_bt::bcast(t, mm), b);
+    for (int c = 0; c < RW; ++c) o[c] = p[c];
+  };
+  load_red(ql - 1);
+  for (int64_t q = ql - 1; q >= q0; --q) {
+    double bt[2] = {o[0], o[1 + NV]};
+    double g[NV], h[NV];
+#pragma unroll
+    for (int c = 0; c < NV; ++c) {
+      g[c] = o[1 + c];
+      h[c] = o[2 + NV + c];
+    }
+    if (q > q0) load_red(q - 1);
+    dot_row16<NV, 0>(bt, t, g, h);
     const int64_t j = j0 + (q - q0);
-    if (active) {
-      Z[j * N2 + r] = b;
+    if (writer) {
+      Z[j * N2 + r] = bt[0];
       Z[j * N2 + NV + r] = t;
     }
-    if (q > q0) {
-      double tn = o[1 + NV];
-#pragma unroll
-      for (int mm = 0; mm < NV; ++mm)
-        tn = fma(o[2 + NV + mm], pyro_bt::bcast(t, mm), tn);
-      t = tn;
-    }
+    t = bt[1];
   }
   if (singular && lane == 0 && n_singular) atomicAdd(n_singular, 1);
 }
@@ -360,6 +510,58 @@ k_spike_recover(const double* __restrict__ fact,
 #pragma unroll
       for (int c = 0; c < MW; ++c) fc[c] = fnext[c];
     }
+  }
+}
+
+// (w[0], w[1]) += (v . x, u . y), entry M of x and y in lane M of the group
+template <int NV, int M>
+__device__ __forceinline__ void dot2_row16(double (&w)[2], double x, double y,
+                                           const double (&v)[NV],
+                                           const double (&u)[NV]) {
+  fmac_bcast_2<M>(w[0], x, v[M], w[1], y, u[M]);
+  if constexpr (M + 1 < NV) dot2_row16<NV, M + 1>(w, x, y, v, u);
+}
+
+// The recovery for NV <= 16, four partitions per wave (one per 16-lane
+// group): reading the factors, 8 NV (2 NV + 1) bytes per row, bounds it.
+template <int NV>
+__global__ void __launch_bounds__(64)
+k_spike_recover_grp(const double* __restrict__ fact,
+                    const int64_t* __restrict__ pstart,
+                    const int64_t* __restrict__ pend, int64_t nparts,
+                    const int64_t* __restrict__ jbefore,
+                    const int64_t* __restrict__ jafter,
+                    const double* __restrict__ Z, double* __restrict__ X) {
+  constexpr int MW = 2 * NV + 1;
+  constexpr int N2 = 2 * NV;
+  const int lane = threadIdx.x;
+  const int gl = lane & 15;
+  const int64_t part = static_cast<int64_t>(blockIdx.x) * 4 + (lane >> 4);
+  if (part >= nparts) return;  // whole 16-lane groups leave together
+  const int r = gl < NV ? gl : 0;
+  const int64_t s = pstart[part], e = pend[part];
+  const int64_t jb = jbefore[part], ja = jafter[part];
+  const double xs = jb >= 0 ? Z[jb * N2 + r] : 0.0;       // b_{q-1}
+  double xn = ja >= 0 ? Z[ja * N2 + NV + r] : 0.0;        // t_{q+1}
+  double fc[MW];
+  auto load = [&](int64_t i) {
+    const double* f = fact + (i * NV + r) * MW;
+#pragma unroll
+    for (int c = 0; c < MW; ++c) fc[c] = f[c];
+  };
+  load(e - 1);
+  for (int64_t i = e - 1; i >= s; --i) {
+    // two sums, so that the chain through x_{i+1} is the shorter
+    double u[NV], v[NV], w[2] = {fc[NV], 0.0};
+#pragma unroll
+    for (int c = 0; c < NV; ++c) {
+      u[c] = -fc[c];
+      v[c] = fc[NV + 1 + c];
+    }
+    if (i > s) load(i - 1);
+    dot2_row16<NV, 0>(w, xs, xn, v, u);
+    xn = w[0] + w[1];
+    if (gl < NV) X[i * NV + r] = xn;
   }
 }
 

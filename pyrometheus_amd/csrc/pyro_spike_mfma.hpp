@@ -66,14 +66,6 @@ __device__ __forceinline__ double row16_max_abs(double v) {
   return v;
 }
 
-// Orders this wave's LDS accesses for the compiler (the hardware executes a
-// wave's LDS instructions in order; wave-local data needs no barrier).
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // Workgroup barrier for LDS data only: waits for this wave's LDS accesses,
 // not for its global loads, so the next block's prefetch stays in flight.
 __device__ __forceinline__ void lds_barrier() {
@@ -661,8 +653,13 @@ int solve(const double* L, const double* C, const double* U, const double* R,
                 maps, roff, red, Z, n_singular);
     }
   }
-  k_spike_recover<NV><<<static_cast<unsigned>(nparts), 64, 0, stream>>>(
-      fact, pstart, pend, jbefore, jafter, Z, X);
+  if constexpr (NV <= 16)
+    k_spike_recover_grp<NV><<<static_cast<unsigned>((nparts + 3) / 4), 64, 0,
+                              stream>>>(fact, pstart, pend, nparts, jbefore,
+                                        jafter, Z, X);
+  else
+    k_spike_recover<NV><<<static_cast<unsigned>(nparts), 64, 0, stream>>>(
+        fact, pstart, pend, jbefore, jafter, Z, X);
   return pyro::launch_status();
 }
 
