@@ -227,10 +227,11 @@ class HipLibrary:
         return name in self.functions
 
     def call(self, name: str, *args) -> int:
-        fn = self.functions.get(name)
-        if fn is None:
+        try:
+            fn = self.functions[name]
+        except KeyError:
             raise HipError(f"{os.path.basename(self.path)} does not export "
-                           f"{name}")
+                           f"{name}") from None
         st = fn(*args)
         if st < 0:
             raise HipError(f"{name} failed with status {st}")

@@ -41,7 +41,10 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device, as its raw handle (the
+    ``torch.cuda.Stream`` object that ``current_stream()`` builds around it
+    takes longer than the rest of a small call's checks together)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 class ThermochemistryBase:
@@ -70,10 +73,19 @@ class ThermochemistryBase:
                                               dtype=torch.float64,
                                               device=self.device)
         self.inv_molecular_weights = 1 / self.molecular_weights
+        # zeroed device counters of get_temperature, at rest between calls
+        self._counters = []
 
     # -- argument plumbing ----------------------------------------------------
     def _cells(self, y: torch.Tensor) -> Tuple[torch.Tensor, Tuple[int, ...]]:
         """Return a (ns, N) view/copy with unit cell stride, and the cell shape."""
+        if type(y) is torch.Tensor and y.dim() == 2 and y.is_cuda \
+                and y.dtype is torch.float64:
+            # the usual argument, already as the kernels read it
+            shape, stride = y.shape, y.stride()
+            if shape[0] == self.num_species and stride[1] == 1 \
+                    and stride[0] >= shape[1]:
+                return y, shape[1:]
         if not isinstance(y, torch.Tensor):
             y = torch.as_tensor(np.asarray(y), dtype=torch.float64,
                                 device=self.device)
@@ -92,6 +104,10 @@ class ThermochemistryBase:
 
     def _scalar_field(self, x, n: int, cell_shape) -> Tuple[torch.Tensor, int]:
         """Per-cell input -> (tensor, stride) with stride 0 for broadcasts."""
+        if type(x) is torch.Tensor and n != 1 and x.dtype is torch.float64 \
+                and x.dim() == 1 and x.shape == cell_shape \
+                and x.is_contiguous():
+            return x, 1
         if isinstance(x, Number):
             return torch.tensor([float(x)], dtype=torch.float64,
                                 device=self.device), 0
@@ -119,6 +135,8 @@ class ThermochemistryBase:
 
     @staticmethod
     def _shape(out: torch.Tensor, rows: Optional[int], cell_shape):
+        if len(cell_shape) == 1:
+            return out
         if rows is None:
             return out.reshape(cell_shape)
         return out.reshape((rows,) + tuple(cell_shape))
@@ -392,12 +410,24 @@ class ThermochemistryBase:
         e, es = self._scalar_field(target, n, cs)
         g, gs = self._scalar_field(t_guess, n, cs)
         out = self._out(None, n)
-        fail = torch.zeros(1, dtype=torch.int32, device=self.device)
+        # a counter is taken by one call at a time (list.pop is atomic) and
+        # comes back only after the call has read it as zero, with its
+        # stream waited for, so whoever takes it next may use any stream
+        try:
+            fail = self._counters.pop()
+        except IndexError:
+            fail = torch.zeros(1, dtype=torch.int32, device=self.device)
         self._lib.call("pyro_temperature", e.data_ptr(), es, g.data_ptr(), gs,
                        yy.data_ptr(), yy.stride(0), out.data_ptr(), n,
                        int(do_energy), mode, float(tol), int(maxit),
                        fail.data_ptr(), None, _stream())
         return self._shape(out, None, cs), fail
+
+    def _check_converged(self, fail):
+        if int(fail.item()) > 0:
+            raise RuntimeError("Temperature iteration failed to converge")
+        if len(self._counters) < 8:
+            self._counters.append(fail)
 
     def get_temperature(self, enthalpy_or_energy, t_guess, y, do_energy=False):
         """Per-lane Newton; raises like the reference when a lane has not
@@ -406,8 +436,7 @@ class ThermochemistryBase:
         energy = do_energy is not False
         t, fail = self._temperature(enthalpy_or_energy, t_guess, y, energy,
                                     0, 1.0e-6, 500)
-        if int(fail.item()) > 0:
-            raise RuntimeError("Temperature iteration failed to converge")
+        self._check_converged(fail)
         return t
 
     def get_temperature_jump_bands(self, mass_fractions, do_energy=True):
@@ -457,8 +486,7 @@ class ThermochemistryBase:
         ``h(T, Y) = h*`` stopping per lane once the step is ``<= tol``."""
         t, fail = self._temperature(enthalpy, temp_init, mass_fractions, False,
                                     1, tol, maxiter)
-        if int(fail.item()) > 0:
-            raise RuntimeError("Temperature iteration failed to converge")
+        self._check_converged(fail)
         return t
 
 
