@@ -5,15 +5,15 @@
 //   mech::kTrVisc[NS][5], mech::kTrCond[NS][5]  species fits in ln T,
 //   mech::kTrDiff[NS*NS][5]                      binary-diffusion fits, the
 //                                                symmetric (i, j) table,
-//   mech::kTrW[NS]                               molecular weights,
-//   mech::kTrWilkeS[NS][NS] = (W_j / W_k)^(1/4),
+//   mech::kTrW4[NS] = W^(1/4),
 //   mech::kTrWilkeD[NS][NS] = 1 / sqrt(8 (1 + W_k / W_j)).
 //
-// One cell per lane.  The double sums over species run with the outer
-// species index k uniform across the wave (a runtime loop whose table rows
-// come through scalar loads) and the inner index fully unrolled over the
-// per-lane arrays (mole fractions and the like), so those stay in
-// registers.
+// One cell per lane.  The double sums over species are fully unrolled over
+// per-lane arrays (mole fractions and the like, in registers) with the
+// tables' entries as literals: with scalar loads every few pairs waited for
+// their constants, which bound both sums (262,144 GRI-3.0 cells:
+// diffusivities 566 -> 293 us, Wilke viscosity with its fewer operations 258 -> 133 us; 30,000 cells
+// 174 -> 70 us).  What bounds them now is FP64 issue.
 #pragma once
 
 #include "pyro_common.hpp"
@@ -31,6 +31,12 @@ __device__ __forceinline__ double poly5(cptr c, double l) {
 // (chem_expr.viscosity_polynomial_expr)
 __device__ __forceinline__ double visc_q(int k, double l) {
   return poly5((cptr)&mech::kTrVisc[k][0], l);
+}
+
+// the same of a species known when compiling, its coefficients literals
+__device__ __forceinline__ double visc_lit(int k, double l) {
+  const auto& c = mech::kTrViscHost[k];
+  return fma(l, fma(l, fma(l, fma(l, c[4], vconst(c[3])), c[2]), c[1]), c[0]);
 }
 
 // sqrt(T) sum b (ln T)^n -- chem_expr.conductivity_polynomial_expr
@@ -93,13 +99,6 @@ __device__ __forceinline__ double mole_fractions(const double* __restrict__ Y,
   return mmw;
 }
 
-// x_k for a wave-uniform k, the same arithmetic as mole_fractions
-__device__ __forceinline__ double mole_fraction(const double* __restrict__ Y,
-                                                int64_t ldY, int64_t i, int k,
-                                                double mmw) {
-  return (((cptr)mech::kInvWMem)[k] * Y[k * ldY + i]) * mmw;
-}
-
 // which: 0 mixture viscosity (Wilke), 1 mixture conductivity, 2 species
 // mixture-averaged mass diffusivities (out (NS, ld)).
 template <int WHICH>
@@ -117,23 +116,27 @@ k_mixture_transport(const double* __restrict__ p, int64_t p_stride,
   if constexpr (WHICH == 0) {
     // sum_k x_k mu_k / phi_k with phi_k = sum_j x_j (1 + sqrt(mu_k / mu_j
     // sqrt(W_j / W_k)))^2 / sqrt(8 (1 + W_k / W_j)); with mu = sqrt(T) q^2
-    // the square root is |q_k| (W_j / W_k)^(1/4) / |q_j|.
-    double u[NS];  // 1 / |q_j|
+    // the square root is (|q_k| / W_k^(1/4)) (W_j^(1/4) / |q_j|): one factor
+    // per species, so that a term takes four operations and one constant.
+    double u[NS];  // W_j^(1/4) / |q_j|
 #pragma unroll
-    for (int j = 0; j < NS; ++j) u[j] = 1.0 / fabs(visc_q(j, l));
-    double acc = 0.0;
+    for (int j = 0; j < NS; ++j)
+      u[j] = mech::kTrW4[j] * recip(fabs(visc_lit(j, l)));
+    double acc = 0.0, lp = l;
+#pragma unroll
     for (int k = 0; k < NS; ++k) {
-      const double qk = fabs(visc_q(k, l));
-      const cptr S = (cptr)&mech::kTrWilkeS[k][0];
-      const cptr D = (cptr)&mech::kTrWilkeD[k][0];
+      // (ln T through an empty asm: the next species' factors are not
+      // computed ahead and kept live)
+      asm volatile("" : "+v"(lp), "+v"(acc));
+      const double qk = fabs(visc_lit(k, lp));
+      const double v = qk * (1.0 / mech::kTrW4[k]);
       double phi = 0.0;
 #pragma unroll
       for (int j = 0; j < NS; ++j) {
-        const double b = fma(qk * S[j], u[j], 1.0);
-        phi = fma(x[j] * b, b * D[j], phi);
+        const double b = fma(v, u[j], 1.0);
+        phi = fma(x[j] * (b * b), mech::kTrWilkeD[k][j], phi);
       }
-      const double xk = mole_fraction(Y, ldY, i, k, mmw);
-      acc += xk * (sqt * (qk * qk)) / phi;
+      acc = fma(x[k] * (sqt * (qk * qk)), recip(phi), acc);
     }
     out[i] = acc;
   } else if constexpr (WHICH == 1) {
@@ -162,14 +165,17 @@ k_mixture_transport(const double* __restrict__ p, int64_t p_stride,
     // ln T and the pair's accumulators pass an empty asm every kTrPin pairs:
     // later pairs' fits and reciprocals are not computed ahead (and kept
     // live beside the 2 NS per-species values)
-    constexpr int kTrPin = 4;
+    constexpr int kTrPin = 2;
     double lp = l;
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
 #pragma unroll
       for (int b = a + 1; b < NS; ++b) {
         if ((b - a - 1) % kTrPin == 0) asm volatile("" : "+v"(lp));
-        const double r = recip(poly5((cptr)&mech::kTrDiff[a * NS + b][0], lp));
+        const auto& c = mech::kTrDiffHost[a * NS + b];
+        const double r = recip(fma(
+            lp, fma(lp, fma(lp, fma(lp, c[4], vconst(c[3])), c[2]), c[1]),
+            c[0]));
         acc[a] = fma(x[b], r, acc[a]);
         acc[b] = fma(x[a], r, acc[b]);
         asm volatile("" : "+v"(acc[b]));
@@ -181,7 +187,7 @@ k_mixture_transport(const double* __restrict__ p, int64_t p_stride,
     for (int k = 0; k < NS; ++k) {
       const double denom = acc[k] * it15;
       const double dkk = pair_diffusivity(k, k, t15, l);
-      const double wk = ((cptr)mech::kTrW)[k];
+      const double wk = mech::kW[k];
       out[k * ld + i] = denom > 0.0
                             ? (mmw - x[k] * wk) / (pr * mmw * denom)
                             : dkk / pr;
