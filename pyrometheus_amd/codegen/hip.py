@@ -193,7 +193,8 @@ class _Writer:
 #: every SIMD busy, 13k of them 1.8 of the 2.0 ms of 2^22 cells.)
 DEFAULT_TUNING = {"pin": True, "pin_every": 3, "kc": "species",
                   "lazy": True, "wdot_waves": 2, "deriv_waves": 0,
-                  "lazy_fence": 1, "order_tries": 8, "wdot_tries": 21, "prefetch": 4,
+                  "lazy_fence": 1, "order_tries": 8, "wdot_tries": 21,
+                  "jvp_tries": 21, "vjp_tries": 8, "prefetch": 4,
                   "zform": True, "jac_groups": 4, "ystash": 39}
 
 
@@ -514,8 +515,9 @@ class _Lowering:
     def third_body(self, r: Reaction, C: str = "C", Ctot: str = "Ctot") -> str:
         """[M] = d Ctot + sum_k (eff_k - d) C_k (chem_expr.py:327-345); with
         ``C``/``Ctot`` naming tangent arrays it gives the tangent of [M]."""
-        if C == "C" and self.body_key(r) in self.m_shared:
-            return self.m_shared[self.body_key(r)][0]
+        if self.body_key(r) in self.m_shared:
+            # ([M], log2 [M], tangent of [M]) as formed once per cell
+            return self.m_shared[self.body_key(r)][0 if C == "C" else 2]
         d = r.default_efficiency
         terms = []
         for sp, eff in r.efficiencies:
@@ -617,6 +619,7 @@ class _Lowering:
             else:
                 w(f"const double er = {er};")
                 w("const double ratio = pyro::exp2p(er);")
+            shared = self.m_shared.get(self.body_key(r))
             w(f"const double M = {self.third_body(r)};")
             w("const double pr = M * ratio;")
             w("const double rpr1 = pyro::recip(1.0 + pr);")
@@ -635,8 +638,9 @@ class _Lowering:
                 w(f"const double sS = {S};")
                 w(f"const double fc = pyro::log2p(sS);")
                 w(f"const double dfc = {dS} * pyro::recip(sS) * {c(1 / ln2)};")
+                lM = shared[1] if shared else "pyro::log2p(M)"
                 w("const double lpr = " + ("pyro::log2p(pr);" if er is None
-                                           else "pyro::log2p(M) + er;"))
+                                           else f"{lM} + er;"))
                 w(f"const double u = lpr + fma(-0.67, fc, {c(-0.4 / LOG10_2)});")
                 w(f"const double nn = fma(-1.27, fc, {c(0.75 / LOG10_2)});")
                 w("const double rden = pyro::recip(fma(-0.14, u, nn));")
@@ -1405,6 +1409,47 @@ def _emit_wdot_jvp(w: _Writer, L: _Lowering):
     w("")
 
 
+def _emit_shared_bodies(w: _Writer, L: _Lowering, tangent: bool):
+    """The total concentration and the [M] sums that several reactions share
+    (with ``tangent`` their tangents too), once per cell, kept with log2 [M]
+    in LDS; fills ``L.m_shared`` with the expressions that read them."""
+    m = L.m
+    keys = L.shared_bodies() if L.tuning.get("share_m", True) else []
+    eff = {key: {L.idx[sp]: e - key[0] for sp, e in key[1]} for key in keys}
+    per = 3 if tangent else 2
+    if keys:
+        w(f"__shared__ double ms[{per * len(keys)}][256];")
+        w("double* msw = &ms[0][threadIdx.x];")
+    w("double Ctot = 0.0" + (", dCtot = 0.0;" if tangent else ";"))
+    for j in range(len(keys)):
+        w(f"double M{j} = 0.0" + (f", dM{j} = 0.0;" if tangent else ";"))
+    for k in range(L.ns):
+        w(f"{{ const double c = kInvW[{k}] * rho * Yg[{k} * ldY + i]; "
+          "Ctot += c;")
+        if tangent:
+            w(f"  const double d = kInvW[{k}] * fma(Yg[{k} * ldY + i], a, "
+              f"sv * Vg[{k} * ldVv + i]); dCtot += d;")
+        for j, e in enumerate(eff.values()):
+            if e.get(k, 0.0) != 0.0:
+                w(f"  M{j} = fma({lit(e[k])}, c, M{j});")
+                if tangent:
+                    w(f"  dM{j} = fma({lit(e[k])}, d, dM{j});")
+        w("}")
+    for j, key in enumerate(keys):
+        w(f"M{j} = fma({lit(key[0])}, Ctot, M{j});")
+        w(f"msw[{per * j} * 256] = M{j};")
+        w(f"msw[{per * j + 1} * 256] = pyro::log2p(M{j});")
+        if tangent:
+            w(f"msw[{per * j + 2} * 256] = fma({lit(key[0])}, dCtot, dM{j});")
+        L.m_shared[key] = tuple(f"msr[{per * j + q} * 256]"
+                                for q in range(per))
+    if keys:
+        w("pyro::lptr msr = (pyro::lptr)msw;")
+        # values read back are not kept in registers meanwhile
+        w('asm volatile("" : "+v"(msr) :: "memory");')
+    return keys, eff
+
+
 def _emit_wdot_jvp_lazy(w: _Writer, L: _Lowering):
     """The forward-mode pass with species opened and closed along
     ``reaction_order`` as in ``_emit_wdot_lazy``: C_k and dC_k loaded, E_k
@@ -1455,17 +1500,12 @@ def _emit_wdot_jvp_lazy(w: _Writer, L: _Lowering):
     w("pyro::gptr Yg = (pyro::gptr)Y;")
     w("pyro::gptr Vg = (pyro::gptr)(vY ? vY : Y);")
     if L.uses_ctot():
-        w("double Ctot = 0.0, dCtot = 0.0;")
-        w("#pragma unroll")
-        w("for (int k = 0; k < NS; ++k) {")
-        w("  Ctot += kInvW[k] * rho * Yg[k * ldY + i];")
-        w("  dCtot += " + dcg.format(k="k") + ";")
-        w("}")
+        _emit_shared_bodies(w, L, tangent=True)
     w("double C[NS], dC[NS], E[NS], hrt[NS], w[NS], dw[NS];")
     L.kinv_f = L.species_kc and L.tuning.get("kinv_f", False)
     if L.kinv_f:
         w("double F[NS];")
-    order = reaction_order(L, L.tuning.get("order_tries", 8))
+    order = reaction_order(L, L.tuning.get("jvp_tries", 8))
     uses = [species_uses(L, r) for r in m.reactions]
     last_w = {}
     for pos, ri in enumerate(order):
@@ -1534,7 +1574,7 @@ def _emit_wdot_jvp_lazy(w: _Writer, L: _Lowering):
     w.ind -= 1
     w("}")
     w("")
-    L.kinv_f = False
+    L.kinv_f, L.m_shared = False, {}
 
 
 def _emit_wdot_vjp(w: _Writer, L: _Lowering):
@@ -1644,16 +1684,18 @@ def _emit_wdot_vjp_lazy(w: _Writer, L: _Lowering):
     w("pyro::gptr Bg = (pyro::gptr)wbp;")
     uses_mbd = any(r.kind in ("three-body", "falloff")
                    and r.default_efficiency != 0.0 for r in m.reactions)
+    shared, eff = [], {}
     if L.uses_ctot():
-        w("double Ctot = 0.0;")
-        w("#pragma unroll")
-        w("for (int k = 0; k < NS; ++k) Ctot += kInvW[k] * rho * Yg[k * ldY + i];")
+        shared, eff = _emit_shared_bodies(w, L, tangent=False)
+        # cotangents of the shared [M], handed to their colliders at the end
+        for j in range(len(shared)):
+            w(f"double mbs{j} = 0.0;")
     w("double y[NS], C[NS], E[NS], hrt[NS], wb[NS], Cb[NS];")
     L.kinv_f = L.species_kc and L.tuning.get("kinv_f", False)
     if L.kinv_f:
         w("double F[NS];")
     w("double tb = 0.0, mbd = 0.0, gr = 0.0;")
-    order = reaction_order(L, L.tuning.get("order_tries", 8))
+    order = reaction_order(L, L.tuning.get("vjp_tries", 8))
     uses = [species_uses(L, r) for r in m.reactions]
     last_c = {}
     for pos, ri in enumerate(order):
@@ -1703,19 +1745,25 @@ def _emit_wdot_vjp_lazy(w: _Writer, L: _Lowering):
                 w(f"Cb[{j}] = fma(-g * kinv, {b}, Cb[{j}]);")
         touched = set(cols)
         if r.kind in ("three-body", "falloff"):
-            w("const double mb = rb * dkfM * delta;")
-            for j, e in L.efficiency_terms(r):
-                w(f"Cb[{j}] = fma({L.c(e)}, mb, Cb[{j}]);")
-                touched.add(j)
-            if r.default_efficiency != 0.0:
-                w(f"mbd = fma({L.c(r.default_efficiency)}, mb, mbd);")
+            key = L.body_key(r)
+            if key in shared:
+                w(f"mbs{shared.index(key)} = fma(rb * dkfM, delta, "
+                  f"mbs{shared.index(key)});")
+            else:
+                w("const double mb = rb * dkfM * delta;")
+                for j, e in L.efficiency_terms(r):
+                    w(f"Cb[{j}] = fma({L.c(e)}, mb, Cb[{j}]);")
+                    touched.add(j)
+                if r.default_efficiency != 0.0:
+                    w(f"mbd = fma({L.c(r.default_efficiency)}, mb, mbd);")
         pending.update(touched)
         w.ind -= 1
         w("}")
         done = sorted(k for k in c_u if last_c[k] == pos)
         if (pos + 1) % L.tuning.get("pin_every", 1) == 0 or done \
                 or pos + 1 == len(order):
-            L.pin(w, [f"Cb[{k}]" for k in sorted(pending)] + ["tb", "mbd"])
+            L.pin(w, [f"Cb[{k}]" for k in sorted(pending)] + ["tb", "mbd"]
+                  + [f"mbs{j}" for j in range(len(shared))])
             pending.clear()
         for k in done:
             w(f"gr = fma(Cb[{k}] * kInvW[{k}], y[{k}], gr);")
@@ -1727,17 +1775,28 @@ def _emit_wdot_vjp_lazy(w: _Writer, L: _Lowering):
         # every Cb_k gets mbd: g_rho through sum_k Y_k / W_k = Ctot / rho,
         # g_Y by a last pass over the stored values (read back through a
         # pointer the optimiser cannot relate to the stores above)
+        # (a shared [M]'s cotangent reaches every species by its default
+        # efficiency and the explicit colliders by the rest; to g_rho it is
+        # mbs [M] / rho)
         w("gr = fma(mbd, Ctot / rho, gr);")
+        for j, key in enumerate(shared):
+            w(f"gr = fma(mbs{j}, {L.m_shared[key][0]} / rho, gr);")
+            w(f"mbd = fma({lit(key[0])}, mbs{j}, mbd);")
         w("if (g_Y) {")
         w.ind += 1
         w("pyro::gmptr gy = (pyro::gmptr)g_Y;")
         w('asm volatile("" : "+s"(gy));')
         for k in range(L.ns):
+            mk = "mbd"
+            for j, key in enumerate(shared):
+                e = eff[key].get(k, 0.0)
+                if e != 0.0:
+                    mk = f"fma({lit(e)}, mbs{j}, {mk})"
             if k in closed:
-                w(f"gy[{k} * ldG + i] = fma(mbd * rho, kInvW[{k}], "
+                w(f"gy[{k} * ldG + i] = fma({mk} * rho, kInvW[{k}], "
                   f"gy[{k} * ldG + i]);")
             else:
-                w(f"gy[{k} * ldG + i] = mbd * rho * kInvW[{k}];")
+                w(f"gy[{k} * ldG + i] = {mk} * rho * kInvW[{k}];")
         w.ind -= 1
         w("}")
     else:
@@ -1749,7 +1808,7 @@ def _emit_wdot_vjp_lazy(w: _Writer, L: _Lowering):
     w.ind -= 1
     w("}")
     w("")
-    L.kinv_f = False
+    L.kinv_f, L.m_shared = False, {}
 
 
 def cache_slots(L: _Lowering):
