@@ -1,35 +1,33 @@
-// The partition sweep of pyro_spike.hpp for 16 < NV <= 63 as a blocked
-// Gauss-Jordan whose trailing updates run on the FP64 matrix cores
-// (v_mfma_f64_16x16x4f64).
+// The partition sweep and the interface recursion of pyro_spike.hpp for
+// 16 < NV <= 63 with their block algebra on the FP64 matrix cores
+// (v_mfma_f64_16x16x4f64), four waves per workgroup.
 //
-// One workgroup of four waves per sweep task (two workgroups fit a CU).
-// The augmented block row [C' | slot | E | x] is held as 16 x 16 tiles in
-// the MFMA accumulator layout: 64 rows (NV used) by 192 columns, C' in
-// columns 0..63, slot in 64..127, E in 128..191 with x in column 128 + NV;
-// unused columns and rows are zero.  Wave w holds column tile w of each of
-// the three blocks (C' tile w, slot tile w + 4, E tile w + 8).  In a tile,
-// lane l and register r hold row (l / 16) + 4 r + 16 rt of row tile rt and
-// column l % 16 (the accumulator layout of the 16x16x4 FP64 MFMA: A[i][k]
-// from lane i + 16 k, B[k][j] from lane j + 16 k, D[(l/16)+4r][l%16] in
-// lane l, register r).
+// A 64 x 64 block (NV used, the rest zero; column NV carries a right-hand
+// side where there is one) is spread by columns: wave w holds the column
+// tile 16 w .. 16 w + 15 as four row tiles in the MFMA accumulator layout:
+// in row tile rt, lane l and register r hold row (l / 16) + 4 r + 16 rt of
+// column 16 w + l % 16.  The layout of the B operand (B[k][j] from lane
+// j + 16 k) is that of one register of it: rows 4 r .. 4 r + 3 of a row
+// tile are acc[rt][r].  So a product A B with B in accumulators needs only
+// its A operand (A[i][k] from lane i + 16 k) from LDS, and the pivot rows of
+// a panel, which are the panel's own rows, are registers of each tile.
 //
-// Per block row: each row is scaled so that its largest |C'| entry is 1;
-// then the C' columns are eliminated in panels of eight.  The wave that
-// holds a panel's columns copies them to one row per lane (through LDS) and
-// reduces them alone by Gauss-Jordan with scaled partial pivoting and
-// virtual pivoting, as pyro_bt::gauss_jordan_dpp (pivot from the DPP
-// max-reduction of pivot_key, reciprocal by v_rcp_f64 and two Newton
-// steps, multiplier 1 - 1/piv on the pivot row).  The eight elementary
-// transforms T_k = I - g_k e_{p_k}^T compose to T = I - W E_P^T (W: 64 x 8,
-// E_P: the pivot rows' unit vectors), accumulated as the panel is reduced
-// (W[:, k] = g_k, W[:, c<k] -= g_k W[p_k, c]).  Every wave then applies T
-// to its tiles, A <- A - W A[P, :], with two MFMAs per 16 x 16 tile: W is
-// the A operand (from LDS), the panel's pivot rows of the tile the B
-// operand (gathered through LDS).  The wave that holds the next panel
-// updates that tile first and reduces the next panel before its other
-// tiles, so one workgroup barrier per panel separates the panels.  The
-// result is the same [I | X] as the unblocked elimination up to rounding;
-// row q ends as logical row lk[q].
+// gj_tiles reduces [A | ...] to [I | X]: rows are scaled by powers of two,
+// then the A columns are eliminated in panels of eight.  The wave that
+// holds a panel copies it to one row per lane and reduces it alone; pivot k
+// is row k unless an unused row's entry is more than kPivotRatio times
+// larger, in which case the two rows are exchanged (in the panel at once, in
+// every tile before the panel is applied).  The eight elementary transforms
+// I - g_k e_k^T compose to T = I - W E_P^T, accumulated as the panel is
+// reduced (W[:, k] = g_k, W[:, c<k] -= g_k W[k, c]), and every wave applies
+// it to its tiles with two MFMAs per 16 x 16 tile.  The wave that holds the
+// next panel updates that tile first and reduces the next panel before its
+// other tiles: one workgroup barrier per panel.
+//
+// The chain of 54 pivots per block row (recip, broadcast, 7 columns each)
+// bounds it.  With pivot rows left in place (a search over all rows per
+// pivot, and the panel's rows gathered through LDS for every tile) a block
+// row of the sweep took about 107k cycles at nv = 54.
 #pragma once
 
 #include "pyro_spike.hpp"
@@ -44,28 +42,6 @@ __device__ __forceinline__ d4 mfma_f64(double a, double b, d4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// Max over each 16-lane row of |v| (DPP rotations within the row).
-__device__ __forceinline__ double row16_max_abs(double v) {
-  v = fabs(v);
-#define PYRO_ROR_FMAX(N)                                                    \
-  {                                                                         \
-    const long long b = __double_as_longlong(v);                            \
-    const int lo = __builtin_amdgcn_mov_dpp(static_cast<int>(b), 0x120 + N, \
-                                            0xF, 0xF, false);               \
-    const int hi = __builtin_amdgcn_mov_dpp(static_cast<int>(b >> 32),      \
-                                            0x120 + N, 0xF, 0xF, false);    \
-    const double o = __longlong_as_double(                                  \
-        (static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));    \
-    v = fmax(v, o);                                                         \
-  }
-  PYRO_ROR_FMAX(8)
-  PYRO_ROR_FMAX(4)
-  PYRO_ROR_FMAX(2)
-  PYRO_ROR_FMAX(1)
-#undef PYRO_ROR_FMAX
-  return v;
-}
-
 // Workgroup barrier for LDS data only: waits for this wave's LDS accesses,
 // not for its global loads, so the next block's prefetch stays in flight.
 __device__ __forceinline__ void lds_barrier() {
@@ -74,28 +50,212 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Per-row tables are kept in the tile order (rt, g, r) of row
-// q = 16 rt + g + 4 r, so that a lane's four rows of a row tile are
-// contiguous.
-__device__ __forceinline__ int trow(int q) {
-  return (q & ~15) | ((q & 3) << 2) | ((q >> 2) & 3);
-}
-
-// LDS of one sweep workgroup (odd strides keep the lanes of an access on
-// distinct banks).
-struct MfmaShared {
-  double W[2][64 * 9];    // panel transform, [row][k], by panel parity
-  double R[4][8 * 17];    // per wave: the pivot rows of one tile, [k][col]
-  double pnl[4][64 * 9];  // per wave: a panel as one row per lane, [row][c]
-  double pf[4][64 * 17];  // per wave: the next block's C rows, [row][col]
-  double xpf[64];         // the next block's right-hand side
-  double smax[4][64];     // row maxima of the C' tiles (tile order)
-  double scl[64];         // row scales (tile order)
-  int kOf[2][64];         // pivot slot of each row in the panel or -1 (tile order)
-  int lk[64];             // logical row of each row (tile order)
+struct alignas(16) TileShared {
+  double W[2][64 * 9];         // panel transform, [row][k], by panel parity
+  double pnl[64 * 9];          // a panel as one row per lane, [row][c]
+  double swap[kMfmaWaves][2][48];  // per wave: the two rows of an exchange
+  int smax[64][kMfmaWaves];    // high words of the rows' largest |A|, per wave
+  int with[2][8];              // row exchanged with pivot row k of the panel
+  int any[2];                  // whether the panel exchanges rows at all
   int singular;
 };
 
+// Max over each 16-lane row of a non-negative 32-bit value.
+__device__ __forceinline__ int row16_max(int v) {
+#define PYRO_ROR_MAX(N)                                                      \
+  {                                                                          \
+    const int o = __builtin_amdgcn_update_dpp(0, v, 0x120 + N, 0xF, 0xF,     \
+                                              true);                         \
+    v = v > o ? v : o;                                                       \
+  }
+  PYRO_ROR_MAX(8)
+  PYRO_ROR_MAX(4)
+  PYRO_ROR_MAX(2)
+  PYRO_ROR_MAX(1)
+#undef PYRO_ROR_MAX
+  return v;
+}
+
+// Reduce panel P (columns 8 P .. of the A tile acc of the wave that calls
+// it) and publish its transform and row exchanges.
+template <int NV, int P>
+__device__ __forceinline__ void tile_panel(const d4 (&acc)[4], int lane,
+                                           TileShared& sh, bool& singular) {
+  constexpr int kBuf = P & 1;
+  constexpr int kCol = 8 * (P & 1);  // the panel's first column in the tile
+  constexpr int kNum = NV - 8 * P < 8 ? NV - 8 * P : 8;
+  const int g = lane >> 4, cl = lane & 15;
+  if (cl >= kCol && cl < kCol + 8) {
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sh.pnl[(16 * rt + g + 4 * r) * 9 + (cl - kCol)] = acc[rt][r];
+  }
+  wave_lds_fence();
+  double pn[8], wr[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    pn[k] = sh.pnl[lane * 9 + k];
+    wr[k] = 0.0;
+  }
+  int any = 0;
+#pragma unroll
+  for (int k = 0; k < kNum; ++k) {
+    const int q = 8 * P + k;
+    int with = q;
+    double piv = bcast(pn[k], q);
+    double inv = pyro::recip(piv);
+    const bool worse = lane > q && lane < NV &&
+                       fabs(pn[k]) > kPivotRatio * fabs(piv);
+    if (__builtin_amdgcn_ballot_w64(worse) != 0ull) {
+      // the largest candidate; worse holds for one, so there is one
+      with = pyro_bt::pivot_lane<NV>(
+          pyro_bt::pivot_key(pn[k], lane >= q && lane < NV, lane), 0ull,
+          1ull << q);
+      const int src = lane == q ? with : lane == with ? q : lane;
+#pragma unroll
+      for (int x = 0; x < 8; ++x) {
+        if (x >= k) pn[x] = __shfl(pn[x], src);
+        if (x < k) wr[x] = __shfl(wr[x], src);
+      }
+      any = 1;
+      piv = bcast(pn[k], q);
+      inv = pyro::recip(piv);
+    }
+    if (lane == 0) sh.with[kBuf][k] = with;
+    singular = singular || !(fabs(piv) > 0.0);
+    const double gk = (lane == q) ? 1.0 - inv : pn[k] * inv;
+#pragma unroll
+    for (int x = k + 1; x < kNum; ++x)
+      pn[x] = fma(-gk, bcast(pn[x], q), pn[x]);
+#pragma unroll
+    for (int x = 0; x < k; ++x) wr[x] = fma(-gk, bcast(wr[x], q), wr[x]);
+    wr[k] = gk;
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) sh.W[kBuf][lane * 9 + k] = wr[k];
+  if (lane == 0) sh.any[kBuf] = any;
+}
+
+// The row exchanges of panel P in this wave's tiles, in the order they were
+// made.
+template <int NV, int NB, int P>
+__device__ __forceinline__ void tile_swaps(d4 (&acc)[NB][4], int wv, int lane,
+                                           TileShared& sh) {
+  constexpr int kBuf = P & 1;
+  constexpr int kNum = NV - 8 * P < 8 ? NV - 8 * P : 8;
+  const int g = lane >> 4, cl = lane & 15;
+#pragma unroll 1
+  for (int k = 0; k < kNum; ++k) {
+    const int q = 8 * P + k;
+    const int w = __builtin_amdgcn_readfirstlane(sh.with[kBuf][k]);
+    if (w == q) continue;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * rt + g + 4 * r;
+        if (row == q || row == w) {
+          double* o = sh.swap[wv][row == q ? 0 : 1];
+#pragma unroll
+          for (int j = 0; j < NB; ++j) o[16 * j + cl] = acc[j][rt][r];
+        }
+      }
+    wave_lds_fence();
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * rt + g + 4 * r;
+        if (row == q || row == w) {
+          const double* o = sh.swap[wv][row == q ? 1 : 0];
+#pragma unroll
+          for (int j = 0; j < NB; ++j) acc[j][rt][r] = o[16 * j + cl];
+        }
+      }
+    wave_lds_fence();
+  }
+}
+
+template <int NV, int NB, int P>
+__device__ __forceinline__ void gj_tiles_from(d4 (&acc)[NB][4], int wv,
+                                              int lane, TileShared& sh,
+                                              bool& singular) {
+  constexpr int kBuf = P & 1;
+  constexpr int kPanels = (NV + 7) / 8;
+  const int g = lane >> 4, cl = lane & 15;
+  if (__builtin_amdgcn_readfirstlane(sh.any[kBuf]))
+    tile_swaps<NV, NB, P>(acc, wv, lane, sh);
+  double aw[4][2];
+#pragma unroll
+  for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      aw[rt][ks] = -sh.W[kBuf][(16 * rt + cl) * 9 + 4 * ks + g];
+  auto apply = [&](int j) {
+    const double b0 = acc[j][P / 2][2 * (P & 1)];
+    const double b1 = acc[j][P / 2][2 * (P & 1) + 1];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+      acc[j][rt] = mfma_f64(aw[rt][0], b0, acc[j][rt]);
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+      acc[j][rt] = mfma_f64(aw[rt][1], b1, acc[j][rt]);
+  };
+  // the A tile: live while it holds a column >= 8 (P + 1)
+  if (16 * wv + 16 > 8 * (P + 1)) apply(0);
+  if constexpr (P + 1 < kPanels) {
+    if (wv == (P + 1) / 2) tile_panel<NV, P + 1>(acc[0], lane, sh, singular);
+  }
+#pragma unroll
+  for (int j = 1; j < NB; ++j) apply(j);
+  lds_barrier();
+  if constexpr (P + 1 < kPanels)
+    gj_tiles_from<NV, NB, P + 1>(acc, wv, lane, sh, singular);
+}
+
+// [A | ...] -> [I | X] as described above; row q of X in row q.  Every wave
+// of the workgroup calls it together; its LDS may be reused after it.
+template <int NV, int NB>
+__device__ __forceinline__ void gj_tiles(d4 (&acc)[NB][4], int wv, int lane,
+                                         TileShared& sh, bool& singular) {
+  static_assert(NB <= 3, "three tiles per wave pass the exchange buffer");
+  const int g = lane >> 4, cl = lane & 15;
+  // rows scaled by 2^-e of their largest |A| entry
+#pragma unroll
+  for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int hi = static_cast<int>(__double_as_longlong(acc[0][rt][r]) >> 32)
+                     & 0x7fffffff;
+      const int mx = row16_max(hi);
+      if (cl == 0) sh.smax[16 * rt + g + 4 * r][wv] = mx;
+    }
+  lds_barrier();
+#pragma unroll
+  for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int4 m = *reinterpret_cast<const int4*>(
+          &sh.smax[16 * rt + g + 4 * r][0]);
+      const int mx = max(max(m.x, m.y), max(m.z, m.w)) >> 20;
+      // 2^(1023 - mx); rows of zeros, infinities or NaN stay as they are
+      const int e = (mx > 0 && mx < 2046) ? 2046 - mx : 1023;
+      const double sc =
+          __longlong_as_double(static_cast<long long>(e) << 52);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[j][rt][r] *= sc;
+    }
+  if (wv == 0) tile_panel<NV, 0>(acc[0], lane, sh, singular);
+  lds_barrier();
+  gj_tiles_from<NV, NB, 0>(acc, wv, lane, sh, singular);
+}
+
+// One sweep over a partition, one workgroup per sweep task (blockIdx = 2
+// partition + (0 down, 1 up)), as k_spike_sweep_waves: acc[0] C', acc[1]
+// slot (the coupling to the next row), acc[2] E (the outside unknown met
+// first) with the right-hand side in column NV.
 template <int NV>
 __global__ void __launch_bounds__(64 * kMfmaWaves, 2)
 k_spike_sweep_mfma(const double* __restrict__ L, const double* __restrict__ C,
@@ -105,11 +265,9 @@ k_spike_sweep_mfma(const double* __restrict__ L, const double* __restrict__ C,
                    const int64_t* __restrict__ pend,
                    const int* __restrict__ psys, double* __restrict__ fact,
                    double* __restrict__ maps, int* __restrict__ n_singular) {
-  static_assert(NV > 16 && NV <= 63, "x sits in column 128 + NV < 192");
+  static_assert(NV > 16 && NV <= 63, "column NV carries the right-hand side");
   constexpr int MW = 2 * NV + 1;
-  constexpr int NP = (NV + 7) / 8;  // panels
-  constexpr int XW = NV / 16;       // the wave holding x (in its E tile)
-  __shared__ MfmaShared sh;
+  __shared__ TileShared sh;
   const int64_t part = blockIdx.x >> 1;
   const bool down = (blockIdx.x & 1) == 0;
   const int lane = threadIdx.x & 63;
@@ -129,14 +287,10 @@ k_spike_sweep_mfma(const double* __restrict__ L, const double* __restrict__ C,
   auto back_coef = [&](int64_t i) -> double {
     return down ? L[i] : U[i - 1];
   };
-  // this lane's column within each 64-column block (the same in C', slot
-  // and E: tile w of each), and its rows
-  const int c = 16 * wv + cl;
+  const int c = 16 * wv + cl;  // this lane's column in each block
   auto rowq = [&](int rt, int r) { return 16 * rt + g + 4 * r; };
 
-  // acc[0] C' tile, acc[1] slot tile, acc[2] E tile (with x)
   d4 acc[3][4];
-  // block row 0: [C | diag(sc) | diag(ec) | r], logical row = row
   {
     const int64_t i = row(0);
     const double sc = slot_coef(i);
@@ -157,173 +311,36 @@ k_spike_sweep_mfma(const double* __restrict__ L, const double* __restrict__ C,
   }
   // the loop below reads acc with no wait for these loads
   __builtin_amdgcn_s_waitcnt(0);
-  const unsigned long long all = (1ull << NV) - 1ull;
   bool singular = false;
-
   for (int64_t t = 0; t < m; ++t) {
     const int64_t i = row(t);
-    // prefetch of the next block's C rows (by row index; permuted after
-    // the elimination) and right-hand side
+    // the next block's rows, in flight during this one (from clamped, valid
+    // addresses; entries outside the block are masked where they are used)
+    // column NV's lanes fetch the right-hand side
     d4 cpre[4] = {};
-    double xpre = 0.0, bpre = 0.0, spre = 0.0;
+    double bpre = 0.0, spre = 0.0;
     const bool more = t + 1 < m;
     if (more) {
       const int64_t i1 = row(t + 1);
-      // every lane loads (from a clamped, valid address: 32-bit offsets
-      // from the block's base); entries outside the block are masked where
-      // they are used
-      const double* cb = C + i1 * NV * NV;
-      const int cc = c < NV ? c : NV - 1;
+      const double* base = c < NV ? C + i1 * NV * NV + c : R + i1 * NV;
+      const int ld = c < NV ? NV : 1;
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int q = rowq(rt, r);
-          cpre[rt][r] = cb[(q < NV ? q : NV - 1) * NV + cc];
-        }
-      // one lane per row: lane l fetches row l (used by the wave holding x)
-      xpre = R[i1 * NV + (lane < NV ? lane : NV - 1)];
+        for (int r = 0; r < 4; ++r)
+          cpre[rt][r] = base[(rowq(rt, r) < NV ? rowq(rt, r) : NV - 1) * ld];
       bpre = back_coef(i);
       spre = slot_coef(i1);
     }
-
-    // ---- row scales: the largest |C'| of each row -> 1 ------------------
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const double mx = row16_max_abs(acc[0][rt][r]);
-        if (cl == 0) sh.smax[wv][16 * rt + 4 * g + r] = mx;
-      }
-    lds_barrier();
-    if (wv == 0) {
-      const int q = lane;  // tile-order index
-      const double mx = fmax(fmax(sh.smax[0][q], sh.smax[1][q]),
-                             fmax(sh.smax[2][q], sh.smax[3][q]));
-      sh.scl[q] = mx > 0.0 ? pyro::recip(mx) : 1.0;
-    }
-    lds_barrier();
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      d4 sc;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sc[r] = sh.scl[16 * rt + 4 * g + r];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) acc[j][rt] *= sc;
-    }
-
-    // ---- blocked Gauss-Jordan over the C' columns -------------------------
-    unsigned long long used = 0ull;
-    // reduce panel p (held by wave p / 2) and publish its transform
-    auto reduce_panel = [&](int p) {
-      const int buf = p & 1;
-      const int c0 = 8 * (p & 1);  // panel's first column in the tile
-      const int np = NV - 8 * p < 8 ? NV - 8 * p : 8;
-      double* pn_l = sh.pnl[wv];
-      if (cl >= c0 && cl < c0 + 8) {
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            pn_l[rowq(rt, r) * 9 + (cl - c0)] = acc[0][rt][r];
-      }
-      wave_lds_fence();
-      double pn[8], wr[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        pn[k] = pn_l[lane * 9 + k];
-        wr[k] = 0.0;
-      }
-      const bool active = lane < NV;
-      int kq = -1;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if (k < np) {
-          const int pv = pyro_bt::pivot_lane<NV>(
-              pyro_bt::pivot_key(pn[k], active && !((used >> lane) & 1ull),
-                                 lane),
-              used, all);
-          used |= 1ull << pv;
-          const double piv = bcast(pn[k], pv);
-          singular = singular || !(fabs(piv) > 0.0);
-          const double inv = pyro::recip(piv);
-          const double gk = (lane == pv) ? 1.0 - inv : pn[k] * inv;
-#pragma unroll
-          for (int x = k + 1; x < 8; ++x)
-            pn[x] = fma(-gk, bcast(pn[x], pv), pn[x]);
-#pragma unroll
-          for (int x = 0; x < k; ++x)
-            wr[x] = fma(-gk, bcast(wr[x], pv), wr[x]);
-          wr[k] = gk;
-          if (lane == pv) kq = k;
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) sh.W[buf][lane * 9 + k] = wr[k];
-      sh.kOf[buf][trow(lane)] = kq;
-      if (kq >= 0) sh.lk[trow(lane)] = 8 * p + kq;
-    };
-    // apply panel p's transform to tile j of this wave (the operands are
-    // read from LDS here, so that nothing of panel p stays live in
-    // registers while the next panel is reduced)
-    auto apply_panel = [&](int p, int j) {
-      const int buf = p & 1;
-      double aw[4][2];
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-          aw[rt][ks] = sh.W[buf][(16 * rt + cl) * 9 + 4 * ks + g];
-      double* rl = sh.R[wv];
-      const int np = NV - 8 * p < 8 ? NV - 8 * p : 8;
-      if (np < 8 && g == 0) {
-        for (int k = np; k < 8; ++k) rl[k * 17 + cl] = 0.0;
-      }
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int k = sh.kOf[buf][16 * rt + 4 * g + r];
-          if (k >= 0) rl[k * 17 + cl] = acc[j][rt][r];
-        }
-      wave_lds_fence();
-      const double b0 = rl[g * 17 + cl], b1 = rl[(4 + g) * 17 + cl];
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        acc[j][rt] = mfma_f64(-aw[rt][0], b0, acc[j][rt]);
-        acc[j][rt] = mfma_f64(-aw[rt][1], b1, acc[j][rt]);
-      }
-      wave_lds_fence();
-    };
-
-    if (wv == 0) reduce_panel(0);
-    lds_barrier();
-#pragma unroll 1
-    for (int p = 0; p < NP; ++p) {
-      used |= __ballot(sh.kOf[p & 1][trow(lane)] >= 0);
-      // the C' tile: live while it holds a column >= 8 (p + 1); the wave
-      // holding panel p + 1 reduces it right after updating that tile
-      if (16 * wv + 16 > 8 * (p + 1)) apply_panel(p, 0);
-      if (p + 1 < NP && wv == (p + 1) / 2) reduce_panel(p + 1);
-      apply_panel(p, 1);
-      apply_panel(p, 2);
-      lds_barrier();
-    }
-    if (singular && lane == 0) sh.singular = 1;
-
-    // ---- outputs of the block row ----------------------------------------
-    int lkr[16];
-#pragma unroll
-    for (int x = 0; x < 16; ++x) lkr[x] = sh.lk[16 * (x >> 2) + 4 * g + (x & 3)];
+    gj_tiles<NV, 3>(acc, wv, lane, sh, singular);
     if (down) {
-      // [X_U | X_r | X_W] of each logical row: slot -> columns 0..NV-1,
-      // x -> NV, E -> NV+1..2NV
+      // [X_U | X_r | X_W]: slot -> columns 0..NV-1, x -> NV, E -> NV+1..2NV
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           if (rowq(rt, r) >= NV) continue;
-          double* f = fact + (i * NV + lkr[4 * rt + r]) * MW;
+          double* f = fact + (i * NV + rowq(rt, r)) * MW;
           if (c < NV) {
             f[c] = acc[1][rt][r];
             f[NV + 1 + c] = acc[2][rt][r];
@@ -333,96 +350,70 @@ k_spike_sweep_mfma(const double* __restrict__ L, const double* __restrict__ C,
         }
     }
     if (!more) break;
-
-    // ---- next block row: C_next[lk] - l X_slot | diag(spre) | -l E | ... --
+    // next block row: C_next - l X_slot | diag(spre) | -l E with r - l x
     const double l = bpre;
-    double* pf = sh.pf[wv];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pf[rowq(rt, r) * 17 + cl] = cpre[rt][r];
-    if (wv == XW) sh.xpf[lane] = xpre;
-    wave_lds_fence();
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const bool live = rowq(rt, r) < NV;
-        const int k = lkr[4 * rt + r];
-        const double cn = (live && c < NV) ? pf[k * 17 + cl] : 0.0;
-        acc[0][rt][r] = fma(-l, acc[1][rt][r], cn);
-        acc[1][rt][r] = (live && c == k) ? spre : 0.0;
-        if (wv == XW && c == NV)
-          acc[2][rt][r] = live ? fma(-l, acc[2][rt][r], sh.xpf[k]) : 0.0;
-        else
-          acc[2][rt][r] *= -l;
+        const int q = rowq(rt, r);
+        const bool live = q < NV;
+        acc[0][rt][r] =
+            (live && c < NV) ? fma(-l, acc[1][rt][r], cpre[rt][r]) : 0.0;
+        acc[1][rt][r] = (live && c == q) ? spre : 0.0;
+        acc[2][rt][r] = fma(-l, acc[2][rt][r],
+                            (live && c == NV) ? cpre[rt][r] : 0.0);
       }
-    wave_lds_fence();
-    // every row of the next block is a pivot of one of its panels, so lk
-    // is rewritten (after the next row-scale barriers) before it is read
   }
   // the partition's map from its last block row:
   //   down: x_{e-1} = X_r + X_W x_{s-1} - X_U x_e
   //   up:   x_s     = X_r + X_V x_e     - X_L x_{s-1}
-  {
-    int lkr[16];
 #pragma unroll
-    for (int x = 0; x < 16; ++x) lkr[x] = sh.lk[16 * (x >> 2) + 4 * g + (x & 3)];
+  for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (rowq(rt, r) >= NV || c > NV) continue;
-        double* mp = maps + ((part * 2 + (down ? 0 : 1)) * NV +
-                             lkr[4 * rt + r]) * MW;
-        if (c == NV) {
-          mp[0] = acc[2][rt][r];
-        } else {
-          // E: coefficient of the outside unknown; slot: minus the next's
-          mp[(down ? 1 : 1 + NV) + c] = acc[2][rt][r];
-          mp[(down ? 1 + NV : 1) + c] = -acc[1][rt][r];
-        }
+    for (int r = 0; r < 4; ++r) {
+      const int q = rowq(rt, r);
+      if (q >= NV || c > NV) continue;
+      double* mp = maps + ((part * 2 + (down ? 0 : 1)) * NV + q) * MW;
+      if (c == NV) {
+        mp[0] = acc[2][rt][r];
+      } else {
+        // E: coefficient of the outside unknown; slot: minus the next's
+        mp[(down ? 1 : 1 + NV) + c] = acc[2][rt][r];
+        mp[(down ? 1 + NV : 1) + c] = -acc[1][rt][r];
       }
-  }
+    }
+  if (singular && lane == 0) sh.singular = 1;
   __syncthreads();
   if (threadIdx.x == 0 && sh.singular && n_singular) atomicAdd(n_singular, 1);
 }
 
-// k_spike_reduced_waves with its three nv x nv products on the FP64 matrix
-// cores: per partition q of a system,
-//   A: [Q | .] = B'_q [G_{q-1} | beta_{q-1}] and [P | .] = B_q [G | beta]
-//      (16 output tiles each, 14 k-steps of v_mfma_f64_16x16x4f64; B'_q and
-//      B_q staged in LDS as the A operands, G read from LDS as the B
-//      operand), then the Gauss-Jordan system [I - Q | D'_q | a' + B' beta]
-//      row by row as before (gj_waves, eight waves);
-//   C: [G_q | beta_q] = [D_q | a_q + B beta] + P [H_q | tau_q] (P from LDS
-//      as the A operand, H from LDS as the B operand).
-// The same recursion as k_spike_reduced_waves up to rounding.
+// k_spike_reduced_waves in the tile layout, one workgroup of four waves per
+// system.  [G | beta] of the partition before stays in accumulators (column
+// NV: beta), so per partition q:
+//   [Q | .] = B'_q [G | beta], [P | .] = B_q [G | beta]  (B', B from LDS),
+//   gj_tiles on [I - Q | D'_q with a' + B' beta] -> [H | tau],
+//   [G | beta] = [D_q | a_q + B beta] + P [H | tau]      (P from LDS).
 template <int NV>
-__global__ void __launch_bounds__(64 * kWaves)
+__global__ void __launch_bounds__(64 * kMfmaWaves)
 k_spike_reduced_mfma(const double* __restrict__ maps,
                      const int64_t* __restrict__ roff,
                      double* __restrict__ red, double* __restrict__ Z,
                      int* __restrict__ n_singular) {
-  static_assert(NV > 16 && NV <= 64, "rows on lanes, 64-row tiles");
-  constexpr int T = Tiles<NV>::T;
-  constexpr int LD = Tiles<NV>::LD;
-  constexpr int XC = Tiles<NV>::XC;
-  static_assert(XC < 64, "beta and tau sit in the fourth column tile");
+  static_assert(NV > 16 && NV <= 63, "column NV carries the right-hand side");
   constexpr int MW = 2 * NV + 1;
   constexpr int N2 = 2 * NV;
   constexpr int RW = 2 * NV + 2;
   constexpr int KS = (NV + 3) / 4;  // k-steps of 4
-  constexpr int LB = NV + 1;        // LDS row stride of B' and B (odd)
-  __shared__ double Gs[NV * LD], Ps[NV * LD], Hs[NV * LD];
-  __shared__ double Bp[NV * LB], Bm[NV * LB];
-  __shared__ GjShared sh;
+  constexpr int LD = 65;            // LDS row stride of the A operands (odd)
+  __shared__ TileShared sh;
+  // A operands, zero outside the NV x NV block
+  __shared__ double Bp[64 * LD], Bm[64 * LD];
   const int sy = blockIdx.x;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, cl = lane & 15;
-  const bool active = lane < NV;
-  const int r = active ? lane : 0;
+  const int c = 16 * wv + cl;
   const int64_t j0 = roff[sy], j1 = roff[sy + 1];
   const int64_t nq = j1 - j0 + 1;
   if (nq < 2) return;  // the whole workgroup leaves
@@ -431,168 +422,120 @@ k_spike_reduced_mfma(const double* __restrict__ maps,
     return maps + ((q * 2 + dir) * NV + row) * MW;
   };
   auto rrow = [&](int64_t q, int row) { return red + (q * NV + row) * RW; };
-  auto col = [&](int t) { return kWaves * t + wv; };
-  // the product tiles of this wave: column tile ct, row tiles rt0, rt0 + 1
-  const int ct = wv & 3;
-  const int rt0 = 2 * (wv >> 2);
-  const int tc = 16 * ct + cl;  // this lane's column in the product tiles
-  for (int idx = threadIdx.x; idx < NV * LD; idx += 64 * kWaves) {
-    Gs[idx] = 0.0;
-    Hs[idx] = 0.0;
-    Ps[idx] = 0.0;
-  }
+  auto rowq = [&](int rt, int r) { return 16 * rt + g + 4 * r; };
+  // column c of [D | a] of a map row
+  auto dcol = [&](const double* mr) { return c < NV ? mr[1 + NV + c] : mr[0]; };
+  for (int idx = threadIdx.x; idx < 64 * LD; idx += 64 * kMfmaWaves)
+    Bp[idx] = Bm[idx] = 0.0;
   if (threadIdx.x == 0) sh.singular = 0;
-  __syncthreads();
-  {
-    const double* md = mrow(q0, 0, r);
-    if (active) {
+  bool singular = false;
+  d4 G[4];
+  auto store_G = [&](int64_t q) {
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
-        const int c = col(t);
-        if (c < NV) {
-          const double v = md[1 + NV + c];
-          Gs[r * LD + c] = v;
-          rrow(q0, r)[1 + c] = v;
-        }
-      }
-      if (wv == 0) {
-        Gs[r * LD + XC] = md[0];
-        rrow(q0, r)[0] = md[0];
-      }
-    }
-  }
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (rowq(rt, r) < NV && c <= NV)
+          rrow(q, rowq(rt, r))[c < NV ? 1 + c : 0] = G[rt][r];
+  };
+#pragma unroll
+  for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      G[rt][r] = (rowq(rt, r) < NV && c <= NV)
+                     ? dcol(mrow(q0, 0, rowq(rt, r))) : 0.0;
+  store_G(q0);
+  // acc += A B over KS k-steps, A in LDS, B a column tile in accumulators
+  auto product = [&](const double* A, const d4 (&B)[4], d4 (&acc)[4]) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)
+        acc[rt] = mfma_f64(A[(16 * rt + cl) * LD + 4 * ks + g],
+                           B[ks / 4][ks % 4], acc[rt]);
+  };
   __syncthreads();
   for (int64_t q = q0 + 1; q < q0 + nq; ++q) {
-    // ---- stage B'_q and B_q (rows of the up and down maps) in LDS --------
-    for (int idx = threadIdx.x; idx < NV * NV; idx += 64 * kWaves) {
+    // B'_q and B_q (rows of the up and down maps) to LDS; D' and D to
+    // registers
+    for (int idx = threadIdx.x; idx < NV * NV; idx += 64 * kMfmaWaves) {
       const int row = idx / NV, k = idx - row * NV;
-      Bp[row * LB + k] = mrow(q, 1, row)[1 + k];
-      Bm[row * LB + k] = mrow(q, 0, row)[1 + k];
+      Bp[row * LD + k] = mrow(q, 1, row)[1 + k];
+      Bm[row * LD + k] = mrow(q, 0, row)[1 + k];
     }
+    d4 acc[2][4], D[4];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool ok = rowq(rt, r) < NV && c <= NV;
+        const int row = ok ? rowq(rt, r) : 0;
+        const double d1 = dcol(mrow(q, 1, row)), d0 = dcol(mrow(q, 0, row));
+        acc[1][rt][r] = ok ? d1 : 0.0;
+        D[rt][r] = ok ? d0 : 0.0;
+      }
     __syncthreads();
-    // ---- A: Q = B' [G | beta], P = B [G | beta] on the matrix cores -------
-    {
-      d4 qa[2] = {}, pa[2] = {};
+    d4 Q[4] = {}, P[4] = {};
+    product(Bp, G, Q);
+    product(Bm, G, P);
+    // [I - Q | D' with a' + B' beta], and D with a + B beta
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int k = 4 * ks + g;
-        const double b = (k < NV && tc <= XC) ? Gs[k * LD + tc] : 0.0;
+    for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int i = 16 * (rt0 + u) + cl;
-          const bool ok = i < NV && k < NV;
-          const double ap = ok ? Bp[i * LB + k] : 0.0;
-          const double am = ok ? Bm[i * LB + k] : 0.0;
-          qa[u] = mfma_f64(ap, b, qa[u]);
-          pa[u] = mfma_f64(am, b, pa[u]);
+      for (int r = 0; r < 4; ++r) {
+        const int row = rowq(rt, r);
+        acc[0][rt][r] = (row < NV && c < NV)
+                            ? ((row == c) ? 1.0 : 0.0) - Q[rt][r] : 0.0;
+        if (c == NV) {
+          acc[1][rt][r] += Q[rt][r];
+          D[rt][r] += P[rt][r];
         }
       }
-      // Q to Hs (H of the previous partition is no longer needed), P and
-      // a + B beta to Ps
+    __syncthreads();  // every wave has read B
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+    for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int row = 16 * (rt0 + u) + g + 4 * jj;
-          if (row < NV && (tc < NV || tc == XC)) {
-            Hs[row * LD + tc] = qa[u][jj];
-            Ps[row * LD + tc] =
-                tc == XC ? mrow(q, 0, row)[0] + pa[u][jj] : pa[u][jj];
-          }
-        }
-    }
-    __syncthreads();
-    double a0[T], ab[1][T];
-    double x = mrow(q, 1, r)[0];
+      for (int r = 0; r < 4; ++r)
+        if (c < NV) Bm[rowq(rt, r) * LD + c] = P[rt][r];
+    gj_tiles<NV, 2>(acc, wv, lane, sh, singular);
+    // (its barriers also order P's stores before the reads below)
 #pragma unroll
-    for (int t = 0; t < T; ++t) {
-      const int c = col(t);
-      a0[t] = (active && c < NV) ? ((c == r) ? 1.0 : 0.0) - Hs[r * LD + c]
-                                 : 0.0;
-      ab[0][t] = (active && c < NV) ? mrow(q, 1, r)[1 + NV + c] : 0.0;
-    }
-    x = (wv == 0 && active) ? x + Hs[r * LD + XC] : 0.0;
-    __syncthreads();  // every wave has read Q before H overwrites it
-    int my_k;
-    gj_waves<NV, T, 1>(a0, ab, x, lane, wv, my_k, sh);
-    if (active) {
-      double* o = rrow(q, my_k);
+    for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
-        const int c = col(t);
-        if (c < NV) {
-          Hs[my_k * LD + c] = ab[0][t];
-          o[2 + NV + c] = ab[0][t];
-        }
-      }
-      if (wv == 0) {
-        Hs[my_k * LD + XC] = x;
-        o[1 + NV] = x;
-      }
-    }
-    __syncthreads();
-    // ---- C: [G_q | beta_q] = [D | a + B beta] + P [H | tau] -------------
-    {
-      d4 ga[2];
+      for (int r = 0; r < 4; ++r)
+        if (rowq(rt, r) < NV && c <= NV)
+          rrow(q, rowq(rt, r))[1 + NV + (c < NV ? 1 + c : 0)] = acc[1][rt][r];
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int row = 16 * (rt0 + u) + g + 4 * jj;
-          double v = 0.0;
-          if (row < NV) {
-            if (tc < NV) v = mrow(q, 0, row)[1 + NV + tc];
-            if (tc == XC) v = Ps[row * LD + XC];
-          }
-          ga[u][jj] = v;
-        }
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int k = 4 * ks + g;
-        const double b = (k < NV && tc <= XC) ? Hs[k * LD + tc] : 0.0;
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int i = 16 * (rt0 + u) + cl;
-          const double a = (i < NV && k < NV) ? Ps[i * LD + k] : 0.0;
-          ga[u] = mfma_f64(a, b, ga[u]);
-        }
-      }
-      __syncthreads();  // every wave has read G_{q-1}'s products (P, H)
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int row = 16 * (rt0 + u) + g + 4 * jj;
-          if (row < NV && (tc < NV || tc == XC)) {
-            Gs[row * LD + tc] = ga[u][jj];
-            rrow(q, row)[tc == XC ? 0 : 1 + tc] = ga[u][jj];
-          }
-        }
-    }
-    __syncthreads();
+    for (int rt = 0; rt < 4; ++rt) G[rt] = D[rt];
+    product(Bm, acc[1], G);
+    store_G(q);
+    __syncthreads();  // every wave has read P before the next B is staged
   }
+  if (singular && lane == 0) sh.singular = 1;
+  __syncthreads();
   if (threadIdx.x == 0 && sh.singular && n_singular) atomicAdd(n_singular, 1);
   if (wv != 0) return;
   // back substitution on wave 0 (the rows of red were written by all the
   // waves before the last barrier); t in natural row order, lane r
+  const bool active = lane < NV;
+  const int r = active ? lane : 0;
   const int64_t ql = q0 + nq - 1;
   double t = rrow(ql, r)[1 + NV];
   for (int64_t q = ql - 1; q >= q0; --q) {
     const double* o = rrow(q, r);
-    double b = o[0];
+    double b = o[0], tn = o[1 + NV];
 #pragma unroll
-    for (int mm = 0; mm < NV; ++mm) b = fma(o[1 + mm], bcast(t, mm), b);
+    for (int mm = 0; mm < NV; ++mm) {
+      const double tm = bcast(t, mm);
+      b = fma(o[1 + mm], tm, b);
+      tn = fma(o[2 + NV + mm], tm, tn);
+    }
     const int64_t j = j0 + (q - q0);
     if (active) {
       Z[j * N2 + r] = b;
       Z[j * N2 + NV + r] = t;
     }
-    if (q > q0) {
-      double tn = o[1 + NV];
-#pragma unroll
-      for (int mm = 0; mm < NV; ++mm) tn = fma(o[2 + NV + mm], bcast(t, mm), tn);
-      t = tn;
-    }
+    t = tn;  // of q0: never used
   }
 }
 
@@ -643,7 +586,7 @@ int solve(const double* L, const double* C, const double* U, const double* R,
         if (sweep_form() == 1) {
           mfma = true;
           k_spike_reduced_mfma<NV>
-              <<<static_cast<unsigned>(nsys), 64 * kWaves, 0, stream>>>(
+              <<<static_cast<unsigned>(nsys), 64 * kMfmaWaves, 0, stream>>>(
                   maps, roff, red, Z, n_singular);
         }
       }
