@@ -113,7 +113,13 @@ __device__ __forceinline__ bool temperature_from_h_tangent(
 // U' = -dt/2 U.  The interior mask m_i is 0 on the two end points.
 // Outputs: rhs (P, NV) = -R (AoS), blocks in place of J, L, U (P,), and
 // optionally R itself (NV, ldp) when r_out != nullptr.
-__global__ void __launch_bounds__(256)
+// Waves of an assembly block (the rows per wave are few enough that a batch
+// of a few thousand 53-species points fills the chip) and the odd row
+// stride of its LDS tile.
+constexpr int kAsmWaves = NV <= 16 ? 4 : 16;
+constexpr int kAsmLd = NV | 1;
+
+__global__ void __launch_bounds__(64 * kAsmWaves)
 k_flamelet_assemble(const double* __restrict__ phi, int64_t ldp,
                     const double* __restrict__ S, int64_t lds,
                     double* __restrict__ J, const double* __restrict__ chi,
@@ -135,8 +141,16 @@ k_flamelet_assemble(const double* __restrict__ phi, int64_t ldp,
                     double* __restrict__ rhs, double* __restrict__ L,
                     double* __restrict__ U, double* __restrict__ r_out,
                     int64_t n) {
-  const int64_t i = cell_index();
-  if (i >= n) return;
+  // 64 points per block, one per lane; the block's waves share the rows, and
+  // the right-hand side, which is stored point by point, passes through LDS
+  // so that whole lines of it are written
+  __shared__ double rs[64 * kAsmLd];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * 64;
+  const int64_t i1 = i0 + lane;
+  const int64_t i = i1 < n ? i1 : n - 1;  // lanes past the end store nothing
+  const bool live = i1 < n;
   const int s = sys[i];
   const bool first = (i == off[s]);
   const bool last = (i == off[s + 1] - 1);
@@ -148,8 +162,7 @@ k_flamelet_assemble(const double* __restrict__ phi, int64_t ldp,
   const int mode = mode0 & 1;
   const bool start = (mode0 & 5) == 5;
   const double hdt = (mode == 1) ? 0.5 * dt[s] : 0.0;
-#pragma unroll
-  for (int v = 0; v < NV; ++v) {
+  for (int v = wv; v < NV; v += kAsmWaves) {
     const double p0 = phi[v * ldp + i];
     double lap;
     if (first || last)
@@ -160,26 +173,36 @@ k_flamelet_assemble(const double* __restrict__ phi, int64_t ldp,
     double r = fma(hc, lap, mask * S[v * lds + i]);
     if (first) r -= bc[(s * 2 + 0) * NV + v];
     if (last) r -= bc[(s * 2 + 1) * NV + v];
-    if (r_out) r_out[v * ldp + i] = r;
+    if (r_out && live) r_out[v * ldp + i] = r;
     if (mode == 1) {
       double pp, rp;
       if (start) {
-        pp = phi[v * ldp + i];
+        pp = p0;
         rp = r;
-        phi_prev[v * ldp + i] = pp;
-        r_prev[v * ldp + i] = rp;
+        if (live) {
+          phi_prev[v * ldp + i] = pp;
+          r_prev[v * ldp + i] = rp;
+        }
       } else {
         pp = phi_prev[v * ldp + i];
         rp = r_prev[v * ldp + i];
       }
-      r = phi[v * ldp + i] - pp - hdt * (r + rp);
+      r = p0 - pp - hdt * (r + rp);
     }
-    rhs[i * NV + v] = -r;
+    rs[lane * kAsmLd + v] = -r;
   }
-  const double lo = last ? 0.0 : 0.5 * chs[i + 1] * la[i + 1];
-  const double up = last ? 0.0 : hc * ci;
-  L[i] = (mode == 1) ? -hdt * lo : lo;
-  U[i] = (mode == 1) ? -hdt * up : up;
+  if (wv == 0 && live) {
+    const double lo = last ? 0.0 : 0.5 * chs[i + 1] * la[i + 1];
+    const double up = last ? 0.0 : hc * ci;
+    L[i] = (mode == 1) ? -hdt * lo : lo;
+    U[i] = (mode == 1) ? -hdt * up : up;
+  }
+  __syncthreads();
+  const int64_t m = (n - i0 < 64 ? n - i0 : 64) * NV;
+  for (int64_t f = threadIdx.x; f < m; f += 64 * kAsmWaves) {
+    const int pt = static_cast<int>(f) / NV, v = static_cast<int>(f) - pt * NV;
+    rhs[i0 * NV + f] = rs[pt * kAsmLd + v];
+  }
 }
 
 // Central blocks in place, one thread per entry of J (P, NV, NV) so that
@@ -235,24 +258,37 @@ k_flamelet_update(double* __restrict__ phi, int64_t ldp,
 // enthalpy row and the species rows: out[2 s] = sum v_h^2, out[2 s + 1] =
 // sum v_Y^2.  One block per system, fixed-order strided partial sums and a
 // fixed reduction tree, so a system's value does not depend on the batch.
-__global__ void __launch_bounds__(256)
+// The sums run over points, each thread its own, so that no entry needs its
+// row worked out.
+constexpr int kNormThreads = 1024;
+
+__global__ void __launch_bounds__(kNormThreads)
 k_system_norm2(const double* __restrict__ x, const int64_t* __restrict__ off,
                double* __restrict__ out) {
-  __shared__ double part[2][256];
+  constexpr int kLanes = 8;  // threads sharing a point's row
+  __shared__ double part[2][kNormThreads];
   const int s = blockIdx.x;
-  const int64_t b = off[s] * NV, e = off[s + 1] * NV;
+  const int64_t b = off[s], e = off[s + 1];
+  const int sub = threadIdx.x % kLanes;
   double ah = 0.0, ay = 0.0;
-  for (int64_t j = b + threadIdx.x; j < e; j += 256) {
-    const double q = x[j] * x[j];
-    if ((j - b) % NV == 0)
-      ah += q;
-    else
-      ay += q;
+  for (int64_t i = b + threadIdx.x / kLanes; i < e;
+       i += kNormThreads / kLanes) {
+#pragma unroll
+    for (int v0 = 0; v0 < NV; v0 += kLanes) {
+      const int v = v0 + sub;
+      if (v < NV) {
+        const double q = x[i * NV + v];
+        if (v == 0)
+          ah = fma(q, q, ah);
+        else
+          ay = fma(q, q, ay);
+      }
+    }
   }
   part[0][threadIdx.x] = ah;
   part[1][threadIdx.x] = ay;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
+  for (int w = kNormThreads / 2; w > 0; w >>= 1) {
     if (threadIdx.x < w) {
       part[0][threadIdx.x] += part[0][threadIdx.x + w];
       part[1][threadIdx.x] += part[1][threadIdx.x + w];
@@ -382,7 +418,8 @@ PYRO_API int pyro_flamelet_assemble(
       !lc || !sys || !off || !bc || !rhs || !L || !U ||
       (modes && (!phi_prev || !r_prev || !dt)))
     return pyro::kInvalidArgument;
-  pyro_fl::k_flamelet_assemble<<<pyro::grid_for(n, 256), 256, 0, stream>>>(
+  pyro_fl::k_flamelet_assemble<<<pyro::grid_for(n, 64),
+                                  64 * pyro_fl::kAsmWaves, 0, stream>>>(
       phi, ldp, S, lds, J, chi, chi0, la, lb, lc, sys, off, bc, modes,
       phi_prev, r_prev, dt, rhs, L, U, r_out, n);
   pyro_fl::k_flamelet_blocks<<<pyro::grid_for(
@@ -417,7 +454,8 @@ PYRO_API int pyro_flamelet_update(double* phi, int64_t ldp, const double* x,
     return pyro::kInvalidArgument;
   if (norm2) {
     if (!off || nsys <= 0) return pyro::kInvalidArgument;
-    pyro_fl::k_system_norm2<<<static_cast<unsigned>(nsys), 256, 0, stream>>>(
+    pyro_fl::k_system_norm2<<<static_cast<unsigned>(nsys),
+                              pyro_fl::kNormThreads, 0, stream>>>(
         x, off, norm2);
   }
   pyro_fl::k_flamelet_update<<<pyro::grid_for(n, 256), 256, 0, stream>>>(

@@ -82,7 +82,27 @@ __device__ __forceinline__ void fmac_bcast(double* acc, const double* src,
 // a[j] += (lane K's a[j]) m for j in [0, N)
 template <int K, int N>
 __device__ __forceinline__ void fmac_bcast_self(double* a, double m) {
-  if constexpr (N >= 8) {
+  if constexpr (N >= 14) {
+    asm("s_nop 1" PYRO_FMB("%0", "%0") PYRO_FMB("%1", "%1")
+        PYRO_FMB("%2", "%2") PYRO_FMB("%3", "%3") PYRO_FMB("%4", "%4")
+        PYRO_FMB("%5", "%5") PYRO_FMB("%6", "%6") PYRO_FMB("%7", "%7")
+        PYRO_FMB("%8", "%8") PYRO_FMB("%9", "%9") PYRO_FMB("%10", "%10")
+        PYRO_FMB("%11", "%11") PYRO_FMB("%12", "%12") PYRO_FMB("%13", "%13")
+        : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]),
+          "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7]), "+&v"(a[8]), "+&v"(a[9]),
+          "+&v"(a[10]), "+&v"(a[11]), "+&v"(a[12]), "+&v"(a[13])
+        : [m] "v"(m), [k] "n"(K));
+    fmac_bcast_self<K, N - 14>(a + 14, m);
+  } else if constexpr (N >= 10) {
+    asm("s_nop 1" PYRO_FMB("%0", "%0") PYRO_FMB("%1", "%1")
+        PYRO_FMB("%2", "%2") PYRO_FMB("%3", "%3") PYRO_FMB("%4", "%4")
+        PYRO_FMB("%5", "%5") PYRO_FMB("%6", "%6") PYRO_FMB("%7", "%7")
+        PYRO_FMB("%8", "%8") PYRO_FMB("%9", "%9")
+        : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]),
+          "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7]), "+&v"(a[8]), "+&v"(a[9])
+        : [m] "v"(m), [k] "n"(K));
+    fmac_bcast_self<K, N - 10>(a + 10, m);
+  } else if constexpr (N >= 8) {
     asm("s_nop 1" PYRO_FMB("%0", "%0") PYRO_FMB("%1", "%1")
         PYRO_FMB("%2", "%2") PYRO_FMB("%3", "%3") PYRO_FMB("%4", "%4")
         PYRO_FMB("%5", "%5") PYRO_FMB("%6", "%6") PYRO_FMB("%7", "%7")
@@ -141,15 +161,18 @@ __device__ __forceinline__ void gj_row16_step(double (&a)[W], int gl,
   double piv = row_bcast<K>(a[K]);
   double inv = pyro::recip(piv);
   if constexpr (K + 1 < NV) {
-    const bool worse = gl > K && gl < NV &&
-                       fabs(a[K]) > kPivotRatio * fabs(piv);
-    if (__builtin_amdgcn_ballot_w64(worse) != 0ull) {
+    // the unused rows after row K, in each group
+    constexpr unsigned long long kLater =
+        0x0001000100010001ull * (((1u << NV) - 1u) & ~((2u << K) - 1u));
+    const bool larger = fabs(a[K]) > kPivotRatio * fabs(piv);
+    if (__builtin_amdgcn_ballot_w64(larger) & kLater) {
       // exchange row K with the largest candidate where one is much larger:
       // those two lanes of the group pass their rows through LDS
       const int lane = threadIdx.x & 63;
       const unsigned best = pyro_bt::row16_max_u32(
           pyro_bt::pivot_key(a[K], gl >= K && gl < NV, lane));
-      const unsigned any = pyro_bt::row16_max_u32(worse ? 1u : 0u);
+      const unsigned any = pyro_bt::row16_max_u32(
+          larger && gl > K && gl < NV ? 1u : 0u);
       const int p = 63 - static_cast<int>(best & 63u) - (lane & 48);
       if (any && best >= 64u && (gl == K || gl == p)) {
         double(&mine)[W] = rows[lane >> 4][gl == K ? 0 : 1];
@@ -168,15 +191,15 @@ __device__ __forceinline__ void gj_row16_step(double (&a)[W], int gl,
   }
   singular = singular || !(fabs(piv) > 0.0);
   const double g = (gl == K) ? inv - 1.0 : -(a[K] * inv);
-  fmac_bcast_self<K, NV - 1 - K>(a + K + 1, g);
   if constexpr (kSlot) {
-    fmac_bcast_self<K, K + 1>(a + NV, g);
+    // columns K+1 .. NV+K (the rest of A and the live slot columns)
+    fmac_bcast_self<K, NV>(a + K + 1, g);
     fmac_bcast_self<K, W - 2 * NV>(a + 2 * NV, g);
     if constexpr (K + 1 < NV) {
       if (full) fmac_bcast_self<K, NV - 1 - K>(a + NV + K + 1, g);
     }
   } else {
-    fmac_bcast_self<K, W - NV>(a + NV, g);
+    fmac_bcast_self<K, W - 1 - K>(a + K + 1, g);
   }
   if constexpr (K + 1 < NV)
     gj_row16_step<NV, W, kSlot, K + 1>(a, gl, rows, full, singular);
@@ -194,6 +217,9 @@ __device__ __forceinline__ void gauss_jordan_row16(double (&a)[W], int gl,
 #pragma unroll
   for (int c = 0; c < W; ++c) a[c] *= sc;
   bool full = !kSlot;
+  // (through an empty asm: the pivots' lane masks are formed where they are
+  // used instead of kept, and spilled, across block rows)
+  asm volatile("" : "+v"(gl));
   gj_row16_step<NV, W, kSlot, 0>(a, gl, rows, full, singular);
 }
 
@@ -458,9 +484,14 @@ k_spike_reduced(const double* __restrict__ maps,
 
 // Recovery: x_i = X_r,i + X_W,i x_{s-1} - X_U,i x_{i+1}, from the last row
 // of the partition up, with x_{s-1} = b_{q-1} and x_e = t_{q+1} taken from
-// the interface solution Z (jbefore/jafter: interface index or -1).
+// the interface solution Z (jbefore/jafter: interface index or -1).  Four
+// waves share a row's sums by columns (a quarter each) and add them through
+// LDS, so that a wave's loads and its chain per row are a quarter as long
+// (one wave per partition: 97 us for the 5k rows of 16 GRI-3.0 flamelets,
+// 200 waves in flight; columns dealt out in turn: 125 us, the quarters'
+// consecutive columns load as 16 bytes).
 template <int NV>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(256)
 k_spike_recover(const double* __restrict__ fact,
                 const int64_t* __restrict__ pstart,
                 const int64_t* __restrict__ pend,
@@ -469,47 +500,48 @@ k_spike_recover(const double* __restrict__ fact,
                 const double* __restrict__ Z, double* __restrict__ X) {
   constexpr int MW = 2 * NV + 1;
   constexpr int N2 = 2 * NV;
+  constexpr int T = (NV + 3) / 4;  // columns per wave
+  __shared__ double sum[2][4][64];
   const int part = blockIdx.x;
-  const int lane = threadIdx.x;
-  const bool active = lane < NV;
-  const int r = active ? lane : 0;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane < NV ? lane : 0;
   const int64_t s = pstart[part], e = pend[part];
   const int64_t jb = jbefore[part], ja = jafter[part];
-  double xs[NV], xe[NV];
+  const double xs = jb >= 0 ? Z[jb * N2 + r] : 0.0;   // b_{q-1}
+  double xn = ja >= 0 ? Z[ja * N2 + NV + r] : 0.0;    // t_{q+1}
+  const int c0 = T * wv;
+  double fu[T], fw[T], fr;
+  auto load = [&](int64_t i) {
+    const double* f = fact + (i * NV + r) * MW;
 #pragma unroll
-  for (int m = 0; m < NV; ++m) {
-    xs[m] = jb >= 0 ? Z[jb * N2 + m] : 0.0;        // b_{q-1}
-    xe[m] = ja >= 0 ? Z[ja * N2 + NV + m] : 0.0;   // t_{q+1}
-  }
-  double xn[NV];
-#pragma unroll
-  for (int m = 0; m < NV; ++m) xn[m] = xe[m];
-  double fc[MW];
-  {
-    const double* f = fact + ((e - 1) * NV + r) * MW;
-#pragma unroll
-    for (int c = 0; c < MW; ++c) fc[c] = f[c];
-  }
+    for (int t = 0; t < T; ++t) {
+      // the last wave may run over into the next columns of the row, which
+      // it does not use
+      fu[t] = f[c0 + t];
+      fw[t] = f[NV + 1 + c0 + (c0 + t < NV ? t : 0)];
+    }
+    fr = f[NV];
+  };
+  load(e - 1);
+  int buf = 0;
   for (int64_t i = e - 1; i >= s; --i) {
-    double fnext[MW];
-    if (i > s) {
-      const double* f = fact + ((i - 1) * NV + r) * MW;
+    double a = wv == 0 ? fr : 0.0, b = 0.0;
 #pragma unroll
-      for (int c = 0; c < MW; ++c) fnext[c] = f[c];
+    for (int t = 0; t < T; ++t) {
+      const int c = c0 + t;  // uniform
+      if (c < NV) {
+        a = fma(fw[t], bcast(xs, c), a);
+        b = fma(-fu[t], bcast(xn, c), b);
+      }
     }
-    double xr = fc[NV];
-#pragma unroll
-    for (int m = 0; m < NV; ++m) {
-      xr = fma(fc[NV + 1 + m], xs[m], xr);
-      xr = fma(-fc[m], xn[m], xr);
-    }
-    if (active) X[i * NV + r] = xr;
-#pragma unroll
-    for (int m = 0; m < NV; ++m) xn[m] = bcast(xr, m);
-    if (i > s) {
-#pragma unroll
-      for (int c = 0; c < MW; ++c) fc[c] = fnext[c];
-    }
+    if (i > s) load(i - 1);
+    sum[buf][wv][lane] = a + b;
+    __syncthreads();
+    xn = (sum[buf][0][lane] + sum[buf][1][lane]) +
+         (sum[buf][2][lane] + sum[buf][3][lane]);
+    if (wv == 0 && lane < NV) X[i * NV + r] = xn;
+    buf ^= 1;
   }
 }
 

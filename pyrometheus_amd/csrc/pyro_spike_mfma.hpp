@@ -51,11 +51,11 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 struct alignas(16) TileShared {
-  double W[2][64 * 9];         // panel transform, [row][k], by panel parity
+  double W[2][64 * 9];         // -W of the panel, [row][k], by panel parity
   double pnl[64 * 9];          // a panel as one row per lane, [row][c]
   double swap[kMfmaWaves][2][48];  // per wave: the two rows of an exchange
   int smax[64][kMfmaWaves];    // high words of the rows' largest |A|, per wave
-  int with[2][8];              // row exchanged with pivot row k of the panel
+  unsigned long long with[2];  // byte k: row exchanged with pivot row k
   int any[2];                  // whether the panel exchanges rows at all
   int singular;
 };
@@ -99,43 +99,52 @@ __device__ __forceinline__ void tile_panel(const d4 (&acc)[4], int lane,
     pn[k] = sh.pnl[lane * 9 + k];
     wr[k] = 0.0;
   }
-  int any = 0;
+  // (lane through an empty asm: the pivots' lane masks are formed where
+  // they are used instead of kept, and spilled, across block rows)
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+  unsigned long long with = 0ull;  // one byte per pivot
+  bool any = false;
 #pragma unroll
   for (int k = 0; k < kNum; ++k) {
     const int q = 8 * P + k;
-    int with = q;
+    // the unused rows after row q
+    const unsigned long long later =
+        ((1ull << NV) - 1ull) & ~((2ull << q) - 1ull);
+    int row = q;
     double piv = bcast(pn[k], q);
     double inv = pyro::recip(piv);
-    const bool worse = lane > q && lane < NV &&
-                       fabs(pn[k]) > kPivotRatio * fabs(piv);
-    if (__builtin_amdgcn_ballot_w64(worse) != 0ull) {
-      // the largest candidate; worse holds for one, so there is one
-      with = pyro_bt::pivot_lane<NV>(
-          pyro_bt::pivot_key(pn[k], lane >= q && lane < NV, lane), 0ull,
-          1ull << q);
-      const int src = lane == q ? with : lane == with ? q : lane;
+    if (__builtin_amdgcn_ballot_w64(fabs(pn[k]) > kPivotRatio * fabs(piv)) &
+        later) {
+      // the largest candidate
+      row = pyro_bt::pivot_lane<NV>(
+          pyro_bt::pivot_key(pn[k], ln >= q && ln < NV, ln), 0ull, 1ull << q);
+      const int src = ln == q ? row : ln == row ? q : ln;
 #pragma unroll
       for (int x = 0; x < 8; ++x) {
         if (x >= k) pn[x] = __shfl(pn[x], src);
         if (x < k) wr[x] = __shfl(wr[x], src);
       }
-      any = 1;
+      any = true;
       piv = bcast(pn[k], q);
       inv = pyro::recip(piv);
     }
-    if (lane == 0) sh.with[kBuf][k] = with;
+    with |= static_cast<unsigned long long>(row) << (8 * k);
     singular = singular || !(fabs(piv) > 0.0);
-    const double gk = (lane == q) ? 1.0 - inv : pn[k] * inv;
+    // wr holds -W
+    const double h = (ln == q) ? inv - 1.0 : -(pn[k] * inv);
 #pragma unroll
-    for (int x = k + 1; x < kNum; ++x)
-      pn[x] = fma(-gk, bcast(pn[x], q), pn[x]);
+    for (int x = k + 1; x < kNum; ++x) pn[x] = fma(h, bcast(pn[x], q), pn[x]);
 #pragma unroll
-    for (int x = 0; x < k; ++x) wr[x] = fma(-gk, bcast(wr[x], q), wr[x]);
-    wr[k] = gk;
+    for (int x = 0; x < k; ++x) wr[x] = fma(h, bcast(wr[x], q), wr[x]);
+    wr[k] = h;
   }
 #pragma unroll
   for (int k = 0; k < 8; ++k) sh.W[kBuf][lane * 9 + k] = wr[k];
-  if (lane == 0) sh.any[kBuf] = any;
+  if (lane == 0) {
+    sh.with[kBuf] = with;
+    sh.any[kBuf] = any;
+  }
 }
 
 // The row exchanges of panel P in this wave's tiles, in the order they were
@@ -146,34 +155,39 @@ __device__ __forceinline__ void tile_swaps(d4 (&acc)[NB][4], int wv, int lane,
   constexpr int kBuf = P & 1;
   constexpr int kNum = NV - 8 * P < 8 ? NV - 8 * P : 8;
   const int g = lane >> 4, cl = lane & 15;
+  const unsigned lo = __builtin_amdgcn_readfirstlane(
+      static_cast<unsigned>(sh.with[kBuf]));
+  const unsigned hi = __builtin_amdgcn_readfirstlane(
+      static_cast<unsigned>(sh.with[kBuf] >> 32));
 #pragma unroll 1
   for (int k = 0; k < kNum; ++k) {
     const int q = 8 * P + k;
-    const int w = __builtin_amdgcn_readfirstlane(sh.with[kBuf][k]);
+    const int w = ((k < 4 ? lo >> (8 * k) : hi >> (8 * (k - 4))) & 255u);
     if (w == q) continue;
+    // register 4 rt + r and lane group of each of the two rows
+    const int qi = (q >> 4) * 4 + ((q >> 2) & 3), wi = (w >> 4) * 4 + ((w >> 2) & 3);
+    const bool mq = g == (q & 3), mw = g == (w & 3);
+    double* sq = sh.swap[wv][0] + cl;
+    double* sw = sh.swap[wv][1] + cl;
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int u = 0; u < 16; ++u) {
+      if (u == qi && mq)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = 16 * rt + g + 4 * r;
-        if (row == q || row == w) {
-          double* o = sh.swap[wv][row == q ? 0 : 1];
+        for (int j = 0; j < NB; ++j) sq[16 * j] = acc[j][u / 4][u % 4];
+      if (u == wi && mw)
 #pragma unroll
-          for (int j = 0; j < NB; ++j) o[16 * j + cl] = acc[j][rt][r];
-        }
-      }
+        for (int j = 0; j < NB; ++j) sw[16 * j] = acc[j][u / 4][u % 4];
+    }
     wave_lds_fence();
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int u = 0; u < 16; ++u) {
+      if (u == qi && mq)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = 16 * rt + g + 4 * r;
-        if (row == q || row == w) {
-          const double* o = sh.swap[wv][row == q ? 1 : 0];
+        for (int j = 0; j < NB; ++j) acc[j][u / 4][u % 4] = sw[16 * j];
+      if (u == wi && mw)
 #pragma unroll
-          for (int j = 0; j < NB; ++j) acc[j][rt][r] = o[16 * j + cl];
-        }
-      }
+        for (int j = 0; j < NB; ++j) acc[j][u / 4][u % 4] = sq[16 * j];
+    }
     wave_lds_fence();
   }
 }
@@ -192,7 +206,7 @@ __device__ __forceinline__ void gj_tiles_from(d4 (&acc)[NB][4], int wv,
   for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
-      aw[rt][ks] = -sh.W[kBuf][(16 * rt + cl) * 9 + 4 * ks + g];
+      aw[rt][ks] = sh.W[kBuf][(16 * rt + cl) * 9 + 4 * ks + g];
   auto apply = [&](int j) {
     const double b0 = acc[j][P / 2][2 * (P & 1)];
     const double b1 = acc[j][P / 2][2 * (P & 1) + 1];
@@ -601,7 +615,7 @@ int solve(const double* L, const double* C, const double* U, const double* R,
                               stream>>>(fact, pstart, pend, nparts, jbefore,
                                         jafter, Z, X);
   else
-    k_spike_recover<NV><<<static_cast<unsigned>(nparts), 64, 0, stream>>>(
+    k_spike_recover<NV><<<static_cast<unsigned>(nparts), 256, 0, stream>>>(
         fact, pstart, pend, jbefore, jafter, Z, X);
   return pyro::launch_status();
 }
