@@ -218,6 +218,32 @@ int pyro_flamelet_assemble(const double* phi, int64_t ldp, const double* S,
                            double* rhs, double* L, double* U, double* r_out,
                            int64_t n, pyro_stream_t stream);
 
+/* pyro_flamelet_assemble without the central blocks. */
+int pyro_flamelet_residual(const double* phi, int64_t ldp, const double* S,
+                           int64_t lds, const double* chi,
+                           const double* chi0, const double* la,
+                           const double* lb, const double* lc, const int* sys,
+                           const int64_t* off, const double* bc,
+                           const int* modes, double* phi_prev,
+                           double* r_prev, const double* dt,
+                           double* rhs, double* L, double* U, double* r_out,
+                           int64_t n, pyro_stream_t stream);
+
+/* pyro_flamelet_source with J written as the central blocks that
+ * pyro_flamelet_assemble would make of it (mechanisms of at most 16
+ * species), so that the blocks are written once. */
+int pyro_flamelet_source_blocks(const double* phi, int64_t ldp,
+                                const double* vd, const double* tguess,
+                                int64_t tg_stride, const double* p,
+                                int64_t p_stride, double* S, int64_t lds,
+                                double* T_out, double* J, const double* chi,
+                                const double* chi0, const double* lb,
+                                const int* sys, const int64_t* off,
+                                const int* modes, const double* dt,
+                                int64_t n, double tol, int maxit,
+                                int* n_fail, int semantics,
+                                pyro_stream_t stream);
+
 /* Block Thomas over B systems whose off-diagonal blocks are L[i] I and
  * U[i] I (the Laplacian coupling), one wavefront per system; X (P, nv).
  * work holds P nv (nv + 1) doubles.  Replaces block_thomas

@@ -122,7 +122,7 @@ constexpr int kAsmLd = NV | 1;
 __global__ void __launch_bounds__(64 * kAsmWaves)
 k_flamelet_assemble(const double* __restrict__ phi, int64_t ldp,
                     const double* __restrict__ S, int64_t lds,
-                    double* __restrict__ J, const double* __restrict__ chi,
+                    const double* __restrict__ chi,
                     const double* __restrict__ chi0,
                     const double* __restrict__ la,
                     const double* __restrict__ lb,
@@ -405,6 +405,26 @@ k_flamelet_adjoint_blocks(double* __restrict__ J,
 // ---------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------
+PYRO_API int pyro_flamelet_residual(
+    const double* phi, int64_t ldp, const double* S, int64_t lds,
+    const double* chi, const double* chi0, const double* la,
+    const double* lb, const double* lc,
+    const int* sys, const int64_t* off, const double* bc, const int* modes,
+    double* phi_prev, double* r_prev, const double* dt,
+    double* rhs, double* L, double* U, double* r_out, int64_t n,
+    hipStream_t stream) {
+  if (n == 0) return pyro::kOk;
+  if (n < 0 || ldp < n || lds < n || !phi || !S || !chi || !la || !lb ||
+      !lc || !sys || !off || !bc || !rhs || !L || !U ||
+      (modes && (!phi_prev || !r_prev || !dt)))
+    return pyro::kInvalidArgument;
+  pyro_fl::k_flamelet_assemble<<<pyro::grid_for(n, 64),
+                                  64 * pyro_fl::kAsmWaves, 0, stream>>>(
+      phi, ldp, S, lds, chi, chi0, la, lb, lc, sys, off, bc, modes,
+      phi_prev, r_prev, dt, rhs, L, U, r_out, n);
+  return pyro::launch_status();
+}
+
 PYRO_API int pyro_flamelet_assemble(
     const double* phi, int64_t ldp, const double* S, int64_t lds, double* J,
     const double* chi, const double* chi0, const double* la,
@@ -414,14 +434,12 @@ PYRO_API int pyro_flamelet_assemble(
     double* rhs, double* L, double* U, double* r_out, int64_t n,
     hipStream_t stream) {
   if (n == 0) return pyro::kOk;
-  if (n < 0 || ldp < n || lds < n || !phi || !S || !J || !chi || !la || !lb ||
-      !lc || !sys || !off || !bc || !rhs || !L || !U ||
-      (modes && (!phi_prev || !r_prev || !dt)))
-    return pyro::kInvalidArgument;
-  pyro_fl::k_flamelet_assemble<<<pyro::grid_for(n, 64),
-                                  64 * pyro_fl::kAsmWaves, 0, stream>>>(
-      phi, ldp, S, lds, J, chi, chi0, la, lb, lc, sys, off, bc, modes,
-      phi_prev, r_prev, dt, rhs, L, U, r_out, n);
+  if (!J) return pyro::kInvalidArgument;
+  const int st = pyro_flamelet_residual(phi, ldp, S, lds, chi, chi0, la, lb,
+                                        lc, sys, off, bc, modes, phi_prev,
+                                        r_prev, dt, rhs, L, U, r_out, n,
+                                        stream);
+  if (st != pyro::kOk) return st;
   pyro_fl::k_flamelet_blocks<<<pyro::grid_for(
                                    n * pyro_fl::NV * pyro_fl::NV, 256),
                                256, 0, stream>>>(J, chi, chi0, lb, sys, off,

@@ -330,6 +330,35 @@ class FlameletBatch:
                       self.rhs.data_ptr(), self.L.data_ptr(),
                       self.U.data_ptr(), _ptr(r_out), self.P, _stream())
 
+    def _source_and_system(self, phi, chi, vd, tguess, p, modes, phi_prev,
+                           r_prev, chi0):
+        """``source`` with its Jacobian and ``assemble`` in the pass that the
+        register-Jacobian kernel allows: the central blocks leave it
+        finished, so they are written once instead of written, read and
+        written again."""
+        phi, chi, phi_prev, r_prev, chi0 = (_rows(x, "input") for x in
+                                            (phi, chi, phi_prev, r_prev,
+                                             chi0))
+        vd, tguess, p = (_rows(x, "input") for x in (vd, tguess, p))
+        dt = self.dt.data_ptr() if modes is not None else None
+        self.n_fail.zero_()
+        self._call("pyro_flamelet_source_blocks", phi.data_ptr(),
+                   phi.stride(0), _ptr(vd), tguess.data_ptr(), 1,
+                   p.data_ptr(), 1, self.S.data_ptr(), self.P,
+                   self.T.data_ptr(), self.J.data_ptr(), chi.data_ptr(),
+                   _ptr(chi0), self.lb.data_ptr(), self.sys.data_ptr(),
+                   self.off.data_ptr(), _ptr(modes), dt, self.P, 1e-10, 100,
+                   self.n_fail.data_ptr(),
+                   1 if self.semantics == "reference" else 0, _stream())
+        self._call("pyro_flamelet_residual", phi.data_ptr(), phi.stride(0),
+                   self.S.data_ptr(), self.P, chi.data_ptr(), _ptr(chi0),
+                   self.la.data_ptr(), self.lb.data_ptr(),
+                   self.lc.data_ptr(), self.sys.data_ptr(),
+                   self.off.data_ptr(), self.bc.data_ptr(), _ptr(modes),
+                   _ptr(phi_prev), _ptr(r_prev), dt, self.rhs.data_ptr(),
+                   self.L.data_ptr(), self.U.data_ptr(), None, self.P,
+                   _stream())
+
     def thomas(self):
         if self.partitioned:
             self._call("pyro_flamelet_thomas_partitioned", self.L.data_ptr(),
@@ -381,8 +410,12 @@ class FlameletBatch:
         ``tguess`` to the temperature of the updated points); returns the
         per-flamelet sums of squares of v, (B, 2) on the device as
         [enthalpy row, species rows], and v (P, nv)."""
-        self.source(phi, vd, tguess, p, jac=True)
-        self.assemble(phi, chi, modes, phi_prev, r_prev, chi0=chi0)
+        if self.dense:
+            self._source_and_system(phi, chi, vd, tguess, p, modes, phi_prev,
+                                    r_prev, chi0)
+        else:
+            self.source(phi, vd, tguess, p, jac=True)
+            self.assemble(phi, chi, modes, phi_prev, r_prev, chi0=chi0)
         self.thomas()
         self.update(phi, active if apply else self.none_active,
                     tguess if (apply and refresh_guess) else None)
