@@ -21,12 +21,12 @@ reference                      generated form
 ``nasa7_conditional``          coefficient select on ``T > T_mid``, Horner
 (``chem_expr.py:51-174``)      (strict ``>``: ``T == T_mid`` takes low)
 ``rate_coefficient_expr``      ``Ea == 0``: ``A*T^b`` (``b`` integer: exact
-(``chem_expr.py:310-324``)     multiplies; else ``A*exp(b ln T)``);
-                               else ``exp(ln A + b ln T - Ta/T)``
+(``chem_expr.py:310-324``)     multiplies); else 2 to the power
+                               ``log2 A + b log2 T - (Ta log2 e)/T``
 ``third_body_efficiencies``    ``d*sum(C) + sum((eff-d)*C_k)``
 (``chem_expr.py:327-345``)
 Troe / Lindemann               ``Fcent``, ``f1`` with the ``Pr > 0`` guard,
-(``chem_expr.py:348-421``)     ``F = 10^(Fcent/(1+f1^2))``
+(``chem_expr.py:348-421``)     ``F = 2^(log2 Fcent/(1+f1^2))``
 ``equilibrium_constants_expr`` ``sum_p nu g - sum_r nu g - dnu*c0``;
 (``chem_expr.py:274-302``)     irreversible placeholder ``-0.17364695002734*T``
 ``rate_of_progress_expr``      ``k_f*(prod C^nu' - exp(-ln K_c) prod C^nu'')``
@@ -110,7 +110,15 @@ class _Writer:
 #:           update, along a reaction order that keeps few species open
 #:           (``reaction_order``); ``order_tries`` greedy restarts
 #:           (``wdot_tries`` for omega-dot: GRI-3.0's peak falls from 73 to
-#:           67 species values at the 21st, 2.40 -> 2.03 ms on 2^22 cells);
+#:           67 species values at the 21st, 2.40 -> 2.03 ms on 2^22 cells,
+#:           and ``jvp_tries``, ``vjp_tries`` likewise for the derivative
+#:           passes: the order of the VJP with the fewest values open is the
+#:           first 8 tries' one);
+#:  share_m -- the derivative passes form a third-body sum that several
+#:           reactions have in common, its log2 and its tangent once per
+#:           cell in LDS instead of once per reaction (JVP of 200,001
+#:           GRI-3.0 cells 547 -> 514 us together with ``jvp_tries``, VJP of
+#:           262,144 cells 528 -> 519 us);
 #:  wdot_waves / deriv_waves -- waves per SIMD the compiler must budget
 #:           registers for in k_wdot / k_wdot_jvp (0: its own choice);
 #:  lazy_fence -- an empty asm with a memory clobber every that many
@@ -523,10 +531,6 @@ class _Lowering:
         D = decimal.Decimal
         return "", self.exponent(db, lo.t_a - hi.t_a,
                                  _DEC.ln(D(lo.A)) - _DEC.ln(D(hi.A)))
-
-    def rate_ratio(self, lo, hi) -> str:
-        fac, ex = self.rate_ratio_parts(lo, hi)
-        return fac if ex is None else f"pyro::exp2p({ex})"
 
     @staticmethod
     def body_key(r: Reaction):

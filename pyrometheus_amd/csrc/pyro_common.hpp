@@ -21,7 +21,6 @@ enum Status : int {
 
 constexpr double kGasConstant = 8314.46261815324;  // J/(kmol K)
 constexpr double kOneAtm = 101325.0;               // Pa
-constexpr double kLn10 = 2.302585092994045684;
 
 // One cell per lane: flat 1-D grid over the cell index.  Launches stay far
 // below 2^31 blocks for any cell count that fits in HBM.

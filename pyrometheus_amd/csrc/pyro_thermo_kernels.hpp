@@ -150,15 +150,6 @@ k_species_state(const double* __restrict__ a, int64_t a_stride,
 // ---------------------------------------------------------------------------
 // kinetics
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void load_conc(const double* __restrict__ rho,
-                                          const double* __restrict__ Y,
-                                          int64_t ldY, int64_t i,
-                                          double (&C)[mech::NS]) {
-  const double r = rho[i];
-#pragma unroll
-  for (int k = 0; k < mech::NS; ++k) C[k] = mech::kInvW[k] * r * Y[k * ldY + i];
-}
-
 // Temperatures at which the products of a reaction's Gibbs factors stay far
 // from overflow and underflow (GRI-3.0: 169 K to beyond 10,000 K).
 __device__ __forceinline__ bool progress_range(double t) {

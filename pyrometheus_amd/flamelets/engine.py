@@ -6,14 +6,15 @@ per-point Laplacian coefficients and dissipation rate, and the scratch the
 kernels need.  One Newton update for every flamelet of the batch is one
 launch sequence:
 
-1. ``pyro_flamelet_source`` -- per point: T(h, Y) by Newton, rho, S and the
-   (nv x nv) source Jacobian (chain rule through the analytic kinetics
-   Jacobian held in registers; mechanisms with at most 16 species), or, for
-   larger mechanisms, ``pyro_temperature`` for T(h, Y) followed by
-   ``pyro_source_jacobian`` (each row evaluated in one pass from T and
-   the concentrations);
-2. ``pyro_flamelet_assemble`` -- residual and block-tridiagonal Jacobian,
-   steady or Crank-Nicolson per flamelet;
+1. ``pyro_flamelet_source_blocks`` -- per point: T(h, Y) by Newton, rho, S
+   and the (nv x nv) source Jacobian (chain rule through the analytic
+   kinetics Jacobian held in registers; mechanisms with at most 16 species)
+   written as finished central blocks, or, for larger mechanisms,
+   ``pyro_temperature`` for T(h, Y) followed by ``pyro_source_jacobian``
+   (each row evaluated in one pass from T and the concentrations);
+2. ``pyro_flamelet_residual`` -- residual and coupling blocks, steady or
+   Crank-Nicolson per flamelet (``pyro_flamelet_assemble``, which turns the
+   source Jacobian into the central blocks as well, for larger mechanisms);
 3. ``pyro_flamelet_thomas_partitioned`` -- block Thomas with the Laplacian
    coupling blocks as scalar multiples of the identity, each flamelet cut
    into partitions swept from both ends and joined through an nv-sized
@@ -350,14 +351,19 @@ class FlameletBatch:
                    self.off.data_ptr(), _ptr(modes), dt, self.P, 1e-10, 100,
                    self.n_fail.data_ptr(),
                    1 if self.semantics == "reference" else 0, _stream())
+        self._residual(phi, chi, modes, phi_prev, r_prev, None, chi0)
+
+    def _residual(self, phi, chi, modes, phi_prev, r_prev, r_out, chi0):
+        """``assemble`` without the central blocks (rows already checked)."""
         self._call("pyro_flamelet_residual", phi.data_ptr(), phi.stride(0),
                    self.S.data_ptr(), self.P, chi.data_ptr(), _ptr(chi0),
                    self.la.data_ptr(), self.lb.data_ptr(),
                    self.lc.data_ptr(), self.sys.data_ptr(),
                    self.off.data_ptr(), self.bc.data_ptr(), _ptr(modes),
-                   _ptr(phi_prev), _ptr(r_prev), dt, self.rhs.data_ptr(),
-                   self.L.data_ptr(), self.U.data_ptr(), None, self.P,
-                   _stream())
+                   _ptr(phi_prev), _ptr(r_prev),
+                   self.dt.data_ptr() if modes is not None else None,
+                   self.rhs.data_ptr(), self.L.data_ptr(),
+                   self.U.data_ptr(), _ptr(r_out), self.P, _stream())
 
     def thomas(self):
         if self.partitioned:
@@ -394,11 +400,14 @@ class FlameletBatch:
                  phi_prev=None, r_prev=None, chi0=None):
         """Steady residual R(phi) into ``out`` (nv, P), with the dissipation
         rate chosen per flamelet by bit 1 of ``modes`` as in ``assemble``
-        (bit 0 changes only the outputs that are not used here).  The block
-        storage is overwritten with values that are not used."""
+        (bit 0 changes only the outputs that are not used here).  The central
+        blocks are left alone."""
         self.source(phi, vd, tguess, p, jac=False)
-        self.assemble(phi, chi, modes, phi_prev, r_prev, r_out=out,
-                      chi0=chi0)
+        phi, chi, phi_prev, r_prev, chi0 = (_rows(x, "input") for x in
+                                            (phi, chi, phi_prev, r_prev,
+                                             chi0))
+        self._residual(phi, chi, modes, phi_prev, r_prev,
+                       _rows(out, "r_out", writable=True), chi0)
         return out
 
     def newton_update(self, phi, chi, vd, tguess, p, modes=None,

@@ -243,6 +243,52 @@ def test_gpu_partitioned_matches_oracle(mech, part_len, sweep, device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mech", ["uiuc", "sandiego", "hong", "gri30"])
+@pytest.mark.parametrize("weight", [0.0, 0.05, 0.3])
+def test_gpu_partitioned_exchanges_rows(mech, weight, device):
+    """The partitioned solve where pivots lie in arbitrary rows: each central
+    block is 4 nv (Q + weight I) + N(0, 1) with Q a random pairing of the
+    rows, so that a block needs exchanges all over (weight 0 and 0.05) or
+    keeps a diagonal within the pivot threshold of the largest entry (0.3).
+    The blocks' condition is at most about 2; tolerance 1e-12 of the
+    solution's largest entry as for the other well-conditioned systems."""
+    import torch
+    from pyrometheus_amd import bundled, get_thermochem_class
+    from pyrometheus_amd.flamelets.engine import FlameletBatch
+    gas = get_thermochem_class(bundled(mech))(device=device)
+    nv = gas.num_species + 1
+    sizes = [3, 9, 41, 33]
+    rng = np.random.default_rng(nv)
+    y = np.zeros(nv - 1)
+    y[-1] = 1.0
+    b = FlameletBatch(gas, [np.linspace(0, 1, n) for n in sizes], y, y,
+                      thomas="partitioned", part_len=4)
+    P = sum(sizes)
+    lv, uv = rng.normal(size=P), rng.normal(size=P)
+    C, r = rng.normal(size=(P, nv, nv)), rng.normal(size=(P, nv))
+    for i in range(P):
+        pairs = rng.permutation(nv)[:nv - nv % 2].reshape(-1, 2)
+        Q = np.eye(nv)
+        Q[pairs[:, 0]], Q[pairs[:, 1]] = (np.eye(nv)[pairs[:, 1]],
+                                          np.eye(nv)[pairs[:, 0]])
+        C[i] += 4 * nv * (Q + weight * np.eye(nv))
+    t = lambda a: torch.tensor(a, dtype=torch.float64, device=device)
+    print(f"[exchanges] {mech} weight={weight}", flush=True)
+    b.L.copy_(t(lv))
+    b.U.copy_(t(uv))
+    b.J.copy_(t(C))
+    b.rhs.copy_(t(r))
+    b.thomas()
+    x, o = b.x.cpu().numpy(), 0
+    for n in sizes:
+        s, k = slice(o, o + n), slice(o, o + n - 1)
+        want = block_thomas(lv[k, None, None] * np.eye(nv), C[s],
+                            uv[k, None, None] * np.eye(nv), r[s])
+        assert np.max(np.abs(x[s] - want)) <= 1e-12 * np.max(np.abs(want)), n
+        o += n
+
+
+@pytest.mark.gpu
 def test_gpu_autotuner_schedule(device):
     """The block-Thomas autotuner times the sequential schedule and the
     partitioned one per alpha on a synthetic batch, keeps the fastest for the

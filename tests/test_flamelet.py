@@ -335,6 +335,61 @@ def test_gpu_general_jacobian_matches_register_form(gas, device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mech", ["sandiego", "uiuc"])
+@pytest.mark.parametrize("modes", [None, (0, 1, 2, 3)])
+@pytest.mark.parametrize("semantics", ["exact", "reference"])
+def test_gpu_fused_blocks_match_separate_passes(mech, modes, semantics,
+                                                device):
+    """Central blocks finished by the source kernel against the source
+    Jacobian followed by the assembly, on sizes that end inside, at and past
+    a wave's 64 points: residual, couplings, source and T bit for bit, the
+    blocks to 4 eps of their largest entry per row (the transform's two
+    roundings)."""
+    import torch
+    from pyrometheus_amd import get_thermochem_class
+    from pyrometheus_amd.flamelets.engine import FlameletBatch
+    g = get_thermochem_class(bundled(mech))(device=device)
+    sizes, ns = [3, 64, 62, 70], g.num_species
+    rng = np.random.default_rng(4)
+    y = np.full(ns, 1.0 / ns)
+    b = FlameletBatch(g, [np.linspace(0, 1, n) for n in sizes], y, y,
+                      semantics=semantics)
+    P = sum(sizes)
+    T = _dev(rng.uniform(400.0, 2200.0, P), device)
+    Y = _dev(rng.dirichlet(np.ones(ns), P).T.copy(), device)
+    phi = torch.cat([g.get_mixture_enthalpy_mass(T, Y)[None], Y]).contiguous()
+    b.set_boundary_enthalpy(float(phi[0, 0]), float(phi[0, -1]))
+    one = lambda lo, hi: _dev(rng.uniform(lo, hi, P), device)
+    chi, chi0, vd = one(1, 50), one(1, 50), one(-1e3, 1e3)
+    p = torch.full_like(chi, ONE_ATM)
+    prev = [phi * 1.01, _dev(rng.normal(size=(ns + 1, P)), device)]
+    md = None
+    if modes is None:
+        prev = [None, None]
+    else:
+        md = torch.tensor(modes, dtype=torch.int32, device=device)
+        b.dt.copy_(_dev(rng.uniform(1e-7, 1e-5, len(sizes)), device))
+    out = []
+    for fused in (False, True):
+        b.J.fill_(float("nan"))
+        pr = [None if v is None else v.clone() for v in prev]
+        if fused:
+            b._source_and_system(phi, chi, vd, T + 5.0, p, md, *pr, chi0)
+        else:
+            b.source(phi, vd, T + 5.0, p, jac=True)
+            b.assemble(phi, chi, md, *pr, chi0=chi0)
+        out.append([v.clone() for v in (b.rhs, b.S, b.T, b.J)]
+                   + [v[:P].clone() for v in (b.L, b.U)])
+    assert int(b.n_fail.item()) == 0
+    for i in (0, 1, 2, 4, 5):
+        assert torch.equal(out[0][i], out[1][i]), i
+    Ja, Jb = out[0][3], out[1][3]
+    top = Ja.abs().amax(dim=2, keepdim=True)
+    assert bool(torch.isfinite(Ja).all())
+    assert float(((Ja - Jb).abs() / top).max()) <= 4 * 2.2e-16
+
+
+@pytest.mark.gpu
 def test_gpu_53_species_flamelets(device):
     """GRI-3.0 flamelets (nv = 54): every flamelet converges, one solved
     alone equals itself in the batch bit for bit, h is linear in Z, the

@@ -353,3 +353,64 @@ def test_mass_average_property(name, device):
     exp = ref.get_mass_average_property(Y, prop)
     scale = ref.get_mass_average_property(Y, np.abs(prop))
     assert np.max(np.abs(got - exp) / scale) < 1e-13
+
+
+def _gibbs_terms(m, T):
+    """Sum of the magnitudes of the terms of g_k(T), (species, T): what the
+    rounding errors of g_k are relative to."""
+    t = np.asarray(T)
+    out = []
+    for sp in m.species:
+        c = np.abs(np.where(t[:, None] > sp.t_mid, sp.high, sp.low)).T
+        out.append(c[0] * (1 + np.abs(np.log(t))) + c[1] / 2 * t
+                   + c[2] / 6 * t ** 2 + c[3] / 12 * t ** 3
+                   + c[4] / 20 * t ** 4 + c[5] / t + c[6])
+    return np.array(out)
+
+
+@pytest.mark.parametrize("name", ["sandiego", "gri30"])
+@pytest.mark.parametrize("n", [1, 255, 257])
+def test_progress_rates_at_range_edges(name, n, device):
+    """Net and reverse rates of progress on both sides of the temperatures
+    between which products of per-species Gibbs factors are used, at those
+    temperatures and at the batch sizes around one block.  Tolerance: 1e-12
+    of the gross rate, and 8 eps of the sum of the magnitudes of the Gibbs
+    terms of either side of the reaction (the exponent's own rounding in two
+    independent evaluations)."""
+    from pyrometheus_amd.codegen.hip import _Lowering, gibbs_range
+    m, gas, ref = setup(name, device)
+    lo, hi = gibbs_range(_Lowering(m))
+    assert lo < 200.0 and hi >= 4000.0
+    edge = [lo, np.nextafter(lo, 0.0), lo - 9.0, lo + 0.5, 1000.0, 1500.0, hi,
+            np.nextafter(hi, 1e9), hi + 400.0]
+    T, p, Y = random_states(m, n, seed=50 + n, inert=_inert(m))
+    T[:] = np.resize(edge, n) if n > 1 else lo - 9.0
+    C = ref.get_concentrations(ref.get_density(p, T, Y), Y)
+    print(f"[progress] {name} n={n}", flush=True)
+    rf = ref.get_fwd_rates_of_progress(T, C)
+    rr = ref.get_rev_rates_of_progress(T, C)
+    nu = np.array([[m.reactant_stoich_coeff(k, i) + m.product_stoich_coeff(k, i)
+                    for k in range(m.n_species)] for i in range(m.n_reactions)])
+    scale = ((np.abs(rf) + np.abs(rr))
+             * (1 + 8 * 2.2e-16 / 1e-12 * (nu @ _gibbs_terms(m, T))))
+    Td, Cd = dev(T, device), dev(C, device)
+    assert scaled_err(host(gas.get_net_rates_of_progress(Td, Cd)),
+                      ref.get_net_rates_of_progress(T, C), scale) < 1e-12
+    assert scaled_err(host(gas.get_rev_rates_of_progress(Td, Cd)), rr,
+                      scale) < 1e-12
+
+
+def test_temperature_call_after_failure(device):
+    """A call that raises leaves nothing behind for the next: targets without
+    a root and solvable ones in turn."""
+    m, gas, ref = setup("sandiego", device)
+    T, _, Y = random_states(m, 65, seed=9, inert=_inert(m))
+    Yd, Td = dev(Y, device), dev(T, device)
+    h = gas.get_mixture_enthalpy_mass(Td, Yd)
+    bad = h.clone()
+    bad[64] = float("nan")
+    for _ in range(3):
+        with pytest.raises(RuntimeError):
+            gas.get_temperature(bad, 900.0, Yd)
+        got = host(gas.get_temperature(h, 900.0, Yd))
+        assert np.max(np.abs(got - T)) <= 1e-9
